@@ -6,15 +6,25 @@
 //
 // Work split: the per-batch prefix, slot numbers and merge-row numbers are
 // block-wide scans; block counts and per-core costs are one item / core per
-// thread; the budget bisection evaluates the greedy fill at every midpoint of
-// the next ten levels of the bisection tree at once (one lane per midpoint),
-// then one thread replays the host's exact bisection path through those
-// results; the fills themselves walk the items in order with the item index
-// uniform across the wave; FA and FD rows are written one core per thread.
+// thread. The greedy fills are what the time goes into (one after another they
+// are a serial walk over the items): a fill walks runs of equal items, not
+// items, so its length is about the cores plus the runs; the budget search
+// evaluates every candidate it may need in one walk, a budget per lane (the
+// doubling search, the first levels of the bisection tree that follows it, and
+// the fill of whole items), then one thread replays the host's exact path
+// through the results; every lane leaves checkpoints of its walk, from which the
+// chosen fill's cursors are recorded by as many lanes at once; and costs below
+// 2^20 blocks are walked in floats (a step is a serial chain of about 20 operations
+// and costs some 300 clocks, so the chain's length is what counts). FA and FD rows
+// are written one core per thread. Measured on MI355X (rebuild, us; before: a
+// walk over the items in 64 bits, four to five walks one after another):
+//   64 x 1 rows, 128 heads, top-k 2048   141 -> 38      23 sequences, 640 ragged rows  281 -> 56
+//   8192 prefill rows, window          3354 -> 128     2000 x 1 ragged rows           924 -> 238
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <string>
+#include <type_traits>
 
 #include "../../include/sas_mi355x.h"
 #include "sas_items.h"
@@ -27,9 +37,11 @@ namespace sasdev {
 
 constexpr int NT = 1024;            // threads of the scheduling workgroup
 constexpr int NWAVE = NT / 64;
-constexpr int BWAVES = 4;           // waves evaluating bisection nodes (one per SIMD)
-constexpr int BNODES = 64 * BWAVES - 1;  // nodes of BLEVELS complete levels
-constexpr int BLEVELS = 8;
+constexpr int BWAVES = 3;           // waves evaluating budgets
+constexpr int BLANES = 64 * BWAVES;
+constexpr int BLEVELS = 7;          // bisection levels of a round: 127 lanes
+constexpr int WHOLE_LANE = 63;      // of the first round: the fill of whole items
+constexpr int NCK = 24;             // checkpoints of a walk
 constexpr int64_t NO_SPLIT = INT64_MAX / 4;
 constexpr int64_t SPLIT_PENALTY = 3;  // same rule and constant as the host scheduler
 
@@ -38,77 +50,184 @@ struct Cursor {
   int32_t j;  // first block not yet assigned inside item i
 };
 
-// The greedy fill of sas_metadata.cpp restated item by item, run by a whole
-// wave: the item index is uniform (its block count is broadcast from a
-// register with v_readlane, one LDS read per 64 items), and each lane fills
-// under its own `budget` in O(1) per item. Per lane: the number of cores,
-// counted until it exceeds `stop_after`. With `ends` (all lanes on one
-// budget) lane 0 records the end cursor of every core, as the host does.
-// The host's loop, item by item: a core that is open (it holds something, so
-// used > 0) either takes the whole item ("fits"), or takes `room` blocks when
-// both parts keep >= min_split, and closes. Then fresh cores: the rest fits in
-// one (it stays open), or the core takes T = max(budget - c_item, min_split)
-// blocks and closes, while at least T + min_split blocks are left -- that run
-// is counted in closed form -- and the last of them takes the remainder,
-// staying open when it fits the budget, closing otherwise.
-__device__ int greedy_wave(const int32_t* nblk, int n, int64_t c, int64_t b, int64_t ms,
-                           int stop_after, Cursor* ends) {
-  const int lane = threadIdx.x & 63;
-  const bool rec = ends != nullptr && lane == 0;
-  int cores = 0;
-  bool open = false, dead = false;
-  int64_t used = 0;
-  for (int i0 = 0; i0 < n; i0 += 64) {
-    const int32_t chunk = i0 + lane < n ? nblk[i0 + lane] : 0;
-    const int lim = n - i0 < 64 ? n - i0 : 64;
+// The items as runs of consecutive items of equal block count: run k holds items
+// start[k] .. start[k + 1] - 1, each of nblk[start[k]] blocks.
+struct Runs {
+  const uint16_t* start;  // [num + 1]
+  const int32_t* nblk;    // per item
+  int num;
+};
+
+// Every lane's state each `stride` steps of a walk (the wave's steps, so a state's
+// run is the same in every lane of it): what recording a fill restarts from.
+struct Checkpoints {
+  uint32_t at[NCK][BLANES];  // items left in the run | cores << 16
+  int32_t room[NCK][BLANES];
+  uint16_t run[NCK][BWAVES];
+  uint16_t num[BWAVES];
+};
+
+// Costs below SMALL are walked in floats, which hold them and their sums and
+// differences exactly: a step is a serial chain, and the float forms of its two
+// floored quotients are the shortest.
+constexpr int64_t SMALL = 1 << 20;
+// 1 / d, at most 2^-20.4 of it too small: x * inv_of(d) for 0 <= x < SMALL is then
+// never above the quotient and less than one below it
+__device__ inline float inv_of(float d) { return __builtin_amdgcn_rcpf(d) * (1.0f - 0x1p-21f); }
+__device__ inline float floor_div(float x, float d, float inv) {
+  const float q = __builtin_floorf(x * inv);
+  return __builtin_fmaf(-q, d, x) >= d ? q + 1.0f : q;
+}
+__device__ inline int64_t inv_of(int64_t) { return 0; }
+__device__ inline int64_t floor_div(int64_t x, int64_t d, int64_t) { return x / d; }
+__device__ inline float less(float x, float k, float d) { return __builtin_fmaf(-k, d, x); }
+__device__ inline int64_t less(int64_t x, int64_t k, int64_t d) { return x - k * d; }
+
+// One lane's greedy fill (sas_metadata.cpp), run by run, under its own budget b and
+// shortest piece ms. `room` is what the open core's budget has left, -1 when no
+// core is open. A step: items that fit the open core go into it together; the item
+// after them closes it, taking `room` less the item cost of its blocks when both
+// parts keep >= ms; the rest L goes to fresh cores: ks of them take
+// T = max(b - c, ms) blocks and close, while at least T + ms blocks are left, and
+// one takes the remainder, staying open when it fits the budget (ks is 0 when the
+// first one does) and closing otherwise. The step is select-only: with a budget
+// per lane some lane takes each side of every condition, and branches would only
+// add their latency to a serial walk.
+template <typename V>
+struct Filler {
+  V c, ms, bc, T, t_inv;
+  V room = -1, cores = 0, left = 0;
+
+  __device__ Filler(V c_, V b, V ms_) : c(c_), ms(ms_), bc(b - c_), T(bc > ms_ ? bc : ms_) {
+    t_inv = inv_of(T);
+  }
+  // FIT: whole items may fit an open core (need <= b); BIG: an item may need
+  // several fresh ones (nb > b - c). on_act(L0, ks, L): the step closes a core.
+  template <bool FIT, bool BIG, typename F>
+  __device__ inline void step(V nb, V need, V need_inv, F&& on_act) {
+    if constexpr (FIT) {
+      const V fit = floor_div(room > 0 ? room : (V)0, need, need_inv);
+      const V t = fit < left ? fit : left;
+      room = less(room, t, need);
+      left -= t;
+    }
+    const bool act = left > 0;
+    const V r = room - c, x = nb - r;
+    const V L0 = (r < x ? r : x) >= ms ? x : nb;
+    V ks = 0, L = L0;
+    if constexpr (BIG) {
+      ks = floor_div(L0 > ms ? L0 - ms : (V)0, T, t_inv);
+      L = less(L0, ks, T);
+    }
+    on_act(act, L0, ks, L);
+    const V rest = bc - L;
+    cores += act ? ks + 1 : (V)0;
+    left -= act ? (V)1 : (V)0;
+    room = act ? (BIG && rest < 0 ? (V)-1 : rest) : room;
+  }
+};
+
+// The number of cores of the lane's fill, counted until it exceeds `stop_after`.
+template <typename V>
+__device__ int greedy_fill(const Runs& rn, int64_t c, int64_t b, int64_t ms, int stop_after,
+                           Checkpoints& ck, int stride) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  Filler<V> f((V)c, (V)b, (V)ms);
+  const V stop = (V)stop_after;
+  int nck = 0, due = 0;
+  auto none = [](bool, V, V, V) {};
+  for (int k0 = 0; k0 < rn.num; k0 += 64) {
+    const int kk = k0 + lane < rn.num ? k0 + lane : rn.num - 1;
+    const int my_start = rn.start[kk], my_end = rn.start[kk + 1];
+    const int my_nb = rn.nblk[my_start];
+    const int lim = rn.num - k0 < 64 ? rn.num - k0 : 64;
     for (int k = 0; k < lim; ++k) {
-      const int i = i0 + k;
-      const int64_t nb = __builtin_amdgcn_readlane(chunk, k);
-      if (dead) continue;
-      int64_t L = nb;
-      if (open) {
-        if (used + c + L <= b) {
-          used += c + L;
-          continue;
+      const V nb = (V)__builtin_amdgcn_readlane(my_nb, k);
+      const V need = f.c + nb;
+      const V need_inv = inv_of(need);
+      f.left = f.cores > stop ? (V)0
+                              : (V)(__builtin_amdgcn_readlane(my_end, k) -
+                                    __builtin_amdgcn_readlane(my_start, k));
+      const bool fit = __ballot(nb <= f.bc) != 0, big = __ballot(nb > f.bc) != 0;
+      auto walk = [&](auto with_fit, auto with_big) {
+        while (__ballot(f.left > 0) != 0) {
+          if (due-- == 0) {
+            // (64-bit walks restart from their beginning)
+            if (nck < (__is_same(V, float) ? NCK : 1)) {
+              ck.at[nck][threadIdx.x] =
+                  (uint32_t)(int)f.left | ((uint32_t)(f.cores > stop ? stop + 1 : f.cores) << 16);
+              ck.room[nck][threadIdx.x] = (int32_t)f.room;
+              if (lane == 0) ck.run[nck][wid] = (uint16_t)(k0 + k);
+              ++nck;
+            }
+            due = stride - 1;
+          }
+          f.template step<decltype(with_fit)::value, decltype(with_big)::value>(nb, need, need_inv,
+                                                                                none);
+          f.left = f.cores > stop ? (V)0 : f.left;
         }
-        const int64_t room = b - used - c;
-        if (room >= ms && L - room >= ms) L -= room;
-        open = false;
-        if (rec) ends[cores - 1] = Cursor{i, (int32_t)(nb - L)};
-      }
-      if (c + L <= b) {  // one fresh core holds the rest
-        if (++cores > stop_after) {
-          dead = true;
-          continue;
-        }
-        open = true;
-        used = c + L;
-        continue;
-      }
-      const int64_t T = b - c > ms ? b - c : ms;
-      // cores that take T and close; when there are any, T < L <= the item's
-      // block count, so the division is a 32-bit one
-      const int64_t ks = L >= T + ms ? (int64_t)((uint32_t)(L - T - ms) / (uint32_t)T) + 1 : 0;
-      if (cores + ks + 1 > stop_after) {
-        cores = stop_after + 1;
-        dead = true;
-        continue;
-      }
-      if (rec)
-        for (int64_t q = 1; q <= ks; ++q) ends[cores + q - 1] = Cursor{i, (int32_t)(nb - L + q * T)};
-      cores += (int)ks + 1;
-      L -= ks * T;
-      if (L <= b - c) {
-        open = true;
-        used = c + L;
-      } else {
-        open = false;
-        if (rec) ends[cores - 1] = Cursor{i + 1, 0};
-      }
+      };
+      if (!big) walk(std::true_type{}, std::false_type{});
+      else if (!fit) walk(std::false_type{}, std::true_type{});
+      else walk(std::true_type{}, std::true_type{});
     }
   }
-  if (!dead && open && rec) ends[cores - 1] = Cursor{n, 0};
-  return cores;
+  if (lane == 0) ck.num[wid] = (uint16_t)nck;
+  return f.cores > stop ? stop_after + 1 : (int)f.cores;
+}
+
+// The end cursors of the fill that lane `who` of the workgroup counted (at most
+// SAS_AIC_CORE_NUM cores): lane l of a wave walks from checkpoint l to the next.
+template <typename V>
+__device__ void record_fill(const Runs& rn, int64_t c, int64_t b, int64_t ms, int who,
+                            const Checkpoints& ck, Cursor* ends) {
+  const int lane = threadIdx.x & 63, nck = ck.num[who >> 6];
+  if (lane >= nck) return;
+  Filler<V> f((V)c, (V)b, (V)ms);
+  auto item_at = [&](int l) {  // the next item of checkpoint l
+    return rn.start[ck.run[l][who >> 6] + 1] - (int)(ck.at[l][who] & 0xFFFFu);
+  };
+  const int n = rn.start[rn.num];
+  const int until = lane + 1 < nck ? item_at(lane + 1) : n;
+  int k = ck.run[lane][who >> 6];
+  f.left = (V)(int)(ck.at[lane][who] & 0xFFFFu);
+  f.cores = (V)(int)(ck.at[lane][who] >> 16);
+  f.room = (V)ck.room[lane][who];
+  int end = rn.start[k + 1];
+  auto record = [&](V core, int i, V j) {
+    if (core <= (V)SAS_AIC_CORE_NUM) ends[(int)core - 1] = Cursor{i, (int32_t)j};
+  };
+  while (end - (int)f.left < until) {
+    if (f.left == 0) {
+      ++k;
+      f.left = (V)(rn.start[k + 1] - end);
+      end = rn.start[k + 1];
+    }
+    const V nb = (V)rn.nblk[rn.start[k]], need = f.c + nb;
+    f.template step<true, true>(nb, need, inv_of(need), [&](bool act, V L0, V ks, V L) {
+      if (!act) return;
+      const int i = end - (int)f.left;
+      if (f.room >= 0) record(f.cores, i, nb - L0);
+      for (V q = 1; q <= ks && f.cores + q <= (V)SAS_AIC_CORE_NUM; q += 1)
+        record(f.cores + q, i, nb - L0 + q * f.T);
+      if (L > f.bc) record(f.cores + 1 + ks, i + 1, 0);
+    });
+  }
+  if (lane == nck - 1 && f.room >= 0) record(f.cores, n, 0);
+}
+
+// [lo, hi] of node `node` (heap order, 1 = root) of the bisection tree over
+// [lo0, hi0]; false when the path to it ends before.
+__device__ inline bool bisect_node(int node, int64_t lo0, int64_t hi0, int64_t* lo, int64_t* hi) {
+  int64_t l = lo0, h = hi0;
+  for (int d = 30 - __clz(node); d >= 0; --d) {
+    if (l >= h) return false;
+    const int64_t mid = l + (h - l) / 2;
+    if ((node >> d) & 1) l = mid + 1; else h = mid;
+  }
+  *lo = l;
+  *hi = h;
+  return l < h;
 }
 
 // cost of core c's range [s, e) (sas_metadata.cpp: makespan, one term)
@@ -163,11 +282,13 @@ constexpr int BPT = (SAS_DEV_SCHED_MAX_BATCH + NT - 1) / NT;  // batches per thr
 __global__ __launch_bounds__(NT) void sched_kernel(const Params p) {
   __shared__ int32_t nblk[SAS_DEV_SCHED_MAX_ITEMS];
   __shared__ int32_t istart[SAS_DEV_SCHED_MAX_BATCH + 1];  // first item of each batch
+  __shared__ uint16_t run_start[SAS_DEV_SCHED_MAX_ITEMS + 1];
+  __shared__ Checkpoints ck;
   __shared__ Cursor ends[SAS_AIC_CORE_NUM];
-  __shared__ uint8_t pred[NT];
+  __shared__ int16_t ncores[BLANES];  // of the last walk, lane by lane
   __shared__ int64_t wsum[2 * NWAVE];
   __shared__ int64_t s_lo, s_hi, s_total, s_longest, s_span;
-  __shared__ int s_err, s_ncore, s_nsplit_ok, s_miss;
+  __shared__ int s_err, s_ncore, s_nwhole, s_miss, s_ks, s_win;
 
   const int tid = threadIdx.x;
   const int wid = tid >> 6;
@@ -291,77 +412,116 @@ __global__ __launch_bounds__(NT) void sched_kernel(const Params p) {
 
   int ncore = 1;
   if (n > 0) {
+    // ---- runs of equal items: thread t looks at items per t .. per (t + 1) - 1 ----
+    const int per = (n + NT - 1) / NT;
+    const int i_lo = per * tid < n ? per * tid : n, i_hi = i_lo + per < n ? i_lo + per : n;
+    auto starts_run = [&](int i) { return i == 0 || nblk[i] != nblk[i - 1]; };
+    int mine = 0;
+    for (int i = i_lo; i < i_hi; ++i) mine += starts_run(i);
+    int64_t num_runs;
+    int at = (int)block_excl_scan(mine, wsum, &num_runs);
+    for (int i = i_lo; i < i_hi; ++i)
+      if (starts_run(i)) run_start[at++] = (uint16_t)i;
+    if (tid == 0) run_start[num_runs] = (uint16_t)n;
+    __syncthreads();
+    const Runs runs = {run_start, nblk, (int)num_runs};
+    // (a budget never exceeds the total of all costs)
+    const bool small = s_total < SMALL && p.min_split_blocks < SMALL;
+    // a walk has at most a step per run and per core: checkpoints cover all of it
+    const int steps = runs.num + p.num_cores + 1;
+    const int stride = steps > 16 * NCK ? (steps + NCK - 1) / NCK : 16;
+    auto clamp_ms = [&](int64_t ms) { return small && ms > SMALL ? SMALL : ms; };
+    auto fill = [&](int64_t b, int64_t ms) -> int {
+      if (small) return greedy_fill<float>(runs, c_item, b, clamp_ms(ms), p.num_cores, ck, stride);
+      return greedy_fill<int64_t>(runs, c_item, b, ms, p.num_cores, ck, stride);
+    };
+    auto record = [&](int64_t b, int64_t ms, int who) {
+      if (small) record_fill<float>(runs, c_item, b, clamp_ms(ms), who, ck, ends);
+      else record_fill<int64_t>(runs, c_item, b, ms, who, ck, ends);
+    };
+    // thread 0: the host's path through evaluated bisection nodes (node 1 is lane
+    // `lane0`); s_win is the lane that counted the fill at s_hi
+    auto replay = [&](int64_t lo, int64_t hi, int lane0) {
+      for (int d = 0, nd = 1; d < BLEVELS && lo < hi; ++d) {
+        const int64_t mid = lo + (hi - lo) / 2;
+        if (ncores[lane0 + nd - 1] <= p.num_cores) {
+          hi = mid;
+          s_win = lane0 + nd - 1;
+          nd = 2 * nd;
+        } else {
+          lo = mid + 1;
+          nd = 2 * nd + 1;
+        }
+      }
+      s_lo = lo;
+      s_hi = hi;
+    };
+
     // ---- smallest budget whose fill fits num_cores (the host's search) ----
-    // doubling search: lane k of wave 0 evaluates h_k = min(total, h_0 2^k)
-    if (wid == 0) {
-      const int64_t h0 = (s_total + p.num_cores - 1) / p.num_cores;
-      int64_t hk = h0 > 1 ? h0 : 1;
-      for (int k = 0; k < (tid & 63) && hk < s_total; ++k) hk = 2 * hk < s_total ? 2 * hk : s_total;
-      const int cores = greedy_wave(nblk, n, c_item, hk, p.min_split_blocks, p.num_cores, nullptr);
-      const bool stop = hk >= s_total || cores <= p.num_cores;
-      const unsigned long long m = __ballot(stop);  // lane 63 reaches total for any total
-      const int ks = __ffsll((long long)m) - 1;
-      const int64_t hi = __shfl(hk, ks);
-      const int64_t prev = __shfl(hk, ks > 0 ? ks - 1 : 0);
-      if (tid == 0) {
-        s_lo = ks > 0 ? prev + 1 : 1;
-        s_hi = hi;
+    // Doubling search: lane k < 63 of wave 0 evaluates h_k = min(total, h_0 2^k),
+    // the last lane the fill of whole items. It mostly ends at h_1, so the waves
+    // beside it evaluate the first levels of the bisection of [h_0 + 1, h_1].
+    const int64_t h0 = (s_total + p.num_cores - 1) / p.num_cores > 1
+                           ? (s_total + p.num_cores - 1) / p.num_cores : 1;
+    const int64_t h1 = 2 * h0 < s_total ? 2 * h0 : s_total;
+    if (wid < BWAVES) {
+      int64_t b = h0, ms = p.min_split_blocks, nlo = 0, nhi = 0;
+      if (tid == WHOLE_LANE) {
+        b = s_longest;
+        ms = NO_SPLIT;
+      } else if (wid == 0) {
+        for (int k = 0; k < tid && b < s_total; ++k) b = 2 * b < s_total ? 2 * b : s_total;
+      } else if (h0 < s_total && tid - 63 < (1 << BLEVELS) &&
+                 bisect_node(tid - 63, h0 + 1, h1, &nlo, &nhi)) {
+        b = nlo + (nhi - nlo) / 2;
+      }
+      const int cores = fill(b, ms);
+      ncores[tid] = (int16_t)cores;
+      if (wid == 0) {
+        const bool stop = tid != WHOLE_LANE && (b >= s_total || cores <= p.num_cores);
+        const int ks = __ffsll((long long)__ballot(stop)) - 1;  // lane 62 has reached total
+        const int64_t hi = __shfl(b, ks);
+        const int64_t prev = __shfl(b, ks > 0 ? ks - 1 : 0);
+        if (tid == 0) {
+          s_lo = ks > 0 ? prev + 1 : 1;
+          s_hi = hi;
+          s_win = s_ks = ks;
+        }
+        if (tid == WHOLE_LANE) s_nwhole = cores;
       }
     }
     __syncthreads();
-    // bisection on [lo, hi]: each round evaluates every midpoint of the next
-    // BLEVELS levels of the bisection tree (one lane per node, one wave per
-    // SIMD), then thread 0 replays the host's path through them
-    for (;;) {
+    if (tid == 0 && s_ks == 1) replay(h0 + 1, h1, 64);
+    __syncthreads();
+    // what is left of [lo, hi], BLEVELS levels a round; then, if the chosen budget
+    // was not counted in the last walk, one more walk at it
+    const bool more = s_lo < s_hi;
+    while (s_lo < s_hi) {
       const int64_t lo = s_lo, hi = s_hi;
-      if (lo >= hi) break;
       if (wid < BWAVES) {
-        const int node = tid + 1;  // heap numbering; depth = floor(log2(node))
-        const int depth = 31 - __clz(node);
-        int64_t l = lo, h = hi;
-        bool live = tid < BNODES;
-        for (int d = depth - 1; d >= 0 && live; --d) {
-          if (l >= h) {
-            live = false;
-            break;
-          }
-          const int64_t mid = l + (h - l) / 2;
-          if ((node >> d) & 1) l = mid + 1; else h = mid;
-        }
-        live = live && l < h;
-        const int64_t mid = live ? l + (h - l) / 2 : hi;  // every lane takes part
-        const int cores = greedy_wave(nblk, n, c_item, mid, p.min_split_blocks, p.num_cores,
-                                      nullptr);
-        if (live) pred[tid] = cores <= p.num_cores;
+        int64_t nlo = 0, nhi = 0, b = hi;
+        if (tid + 1 < (1 << BLEVELS) && bisect_node(tid + 1, lo, hi, &nlo, &nhi))
+          b = nlo + (nhi - nlo) / 2;
+        ncores[tid] = (int16_t)fill(b, p.min_split_blocks);
       }
       __syncthreads();
       if (tid == 0) {
-        int64_t bl = lo, bh = hi;
-        int nd = 1;
-        for (int d = 0; d < BLEVELS && bl < bh; ++d) {
-          const int64_t m = bl + (bh - bl) / 2;
-          if (pred[nd - 1]) {
-            bh = m;
-            nd = 2 * nd;
-          } else {
-            bl = m + 1;
-            nd = 2 * nd + 1;
-          }
-        }
-        s_lo = bl;
-        s_hi = bh;
+        s_win = -1;
+        replay(lo, hi, 0);
       }
       __syncthreads();
     }
-    // ---- the fill at the chosen budget (wave 0) and the no-split count (wave 1) ----
-    if (wid == 0) {
-      const int c = greedy_wave(nblk, n, c_item, s_lo, p.min_split_blocks, SAS_AIC_CORE_NUM, ends);
-      if (tid == 0) s_ncore = c;
-    } else if (wid == 1) {
-      const int c = greedy_wave(nblk, n, c_item, s_longest, NO_SPLIT, p.num_cores, nullptr);
-      if (tid == 64) s_nsplit_ok = c <= p.num_cores;
-    }
-    __syncthreads();
+    // ---- the fill at the chosen budget ----
+    // (a walk of its own only when the last one did not count it)
+    auto walk_and_record = [&](int64_t b, int64_t ms, int who) {
+      if (wid == 0) {
+        if (who < 0) ncores[tid] = (int16_t)fill(b, ms);
+        record(b, ms, who < 0 ? 0 : who);
+        if (tid == 0) s_ncore = ncores[who < 0 ? 0 : who];
+      }
+      __syncthreads();
+    };
+    walk_and_record(s_lo, p.min_split_blocks, s_win);
     ncore = s_ncore;
     int64_t my_span = 0;
     for (int c = tid; c < ncore && ncore <= SAS_AIC_CORE_NUM; c += NT) {
@@ -376,11 +536,8 @@ __global__ __launch_bounds__(NT) void sched_kernel(const Params p) {
     }
     if ((tid & 63) == 0) atomicMax((unsigned long long*)&s_span, (unsigned long long)my_span);
     __syncthreads();
-    if (s_longest <= s_span + SPLIT_PENALTY && s_nsplit_ok && wid == 0) {
-      const int c = greedy_wave(nblk, n, c_item, s_longest, NO_SPLIT, SAS_AIC_CORE_NUM, ends);
-      if (tid == 0) s_ncore = c;
-    }
-    __syncthreads();
+    if (s_longest <= s_span + SPLIT_PENALTY && s_nwhole <= p.num_cores)
+      walk_and_record(s_longest, NO_SPLIT, more || s_win < 0 ? -1 : WHOLE_LANE);
     ncore = s_ncore;
     if (ncore > p.num_cores) {
       if (tid == 0) cfg[1] = -3;  // over capacity
