@@ -113,6 +113,12 @@ int sas_metadata_build_device(int32_t* meta, int batch, const int32_t* act_q,
                               int m_base, int ori_win_left, int scenario, int cmp_ratio,
                               int cmp_topk, int num_cores, int s2_base, int min_split_blocks,
                               int fd_head_chunk, int reuse, void* stream);
+/* The same from the [batch + 1] cumulative query rows (cu_seqlens_q, device). */
+int sas_metadata_build_device_cu(int32_t* meta, int batch, const int32_t* cu_q,
+                                 const int32_t* seqused_kv, int num_heads,
+                                 int m_base, int ori_win_left, int scenario, int cmp_ratio,
+                                 int cmp_topk, int num_cores, int s2_base, int min_split_blocks,
+                                 int fd_head_chunk, int reuse, void* stream);
 
 /* Bytes of split-KV partial workspace for a schedule:
  * num_partial_slots * m_base * (2 * head_dim_v + 8): the partials [slot][head][head_dim_v]
@@ -224,6 +230,25 @@ typedef struct SasAttnArgs {
  * the attention kernel (merge_sync), the split-KV merge kernel on `stream` (a
  * hipStream_t). Asynchronous; no allocation, no host synchronisation. */
 int sas_attention_launch(const SasAttnArgs* args, void* stream);
+
+/* sas_attention_launch with the query rows of the batches in another form than the
+ * q_prefix / act_q_lens arrays (no reference counterpart: api.py:208-240 forms the arrays
+ * on the host), so that a caller launches nothing to form them:
+ * SAS_QLENS_CUMULATIVE: q_prefix is the [batch + 1] cumulative row counts (cu_seqlens_q;
+ *   non-decreasing); act_q_lens is ignored. Rows of out and lse before q_prefix[0] and
+ *   from the schedule's end on (q_prefix[batch] when it covers every batch) are zeroed.
+ * SAS_QLENS_UNIFORM: every batch has total_tokens / batch rows; both arrays are ignored. */
+#define SAS_QLENS_ARRAYS 0
+#define SAS_QLENS_CUMULATIVE 1
+#define SAS_QLENS_UNIFORM 2
+int sas_attention_launch_lens(const SasAttnArgs* args, int q_lens, void* stream);
+
+/* Arrival counters (SasAttnArgs.merge_sync) for calls captured on `stream`, which must be
+ * capturing: a zeroed array of the library's own, the same one for every call of one
+ * capture on one stream. An array belongs to its capture's graph until the process ends;
+ * NULL (see sas_last_error) once SAS_MERGE_SYNC_POOL arrays of the device are taken. */
+#define SAS_MERGE_SYNC_POOL 1024
+uint64_t* sas_merge_sync_take(void* stream);
 
 /* Allocation-free variant of sas_attention_launch (no counterpart in the reference:
  * for callers that cannot allocate device memory, such as code under HIP graph

@@ -37,6 +37,9 @@ SAS_PHASE_PIPELINED = 4        # SasAttnArgs.phases bit: native rows through the
 SAS_PHASE_FP8_QK = 8           # SasAttnArgs.phases bit: fp8 rows, Q·Kᵀ on fp8 MFMA (e4m3 queries)
 SAS_PHASE_ROW_ITEMS = 16       # SasAttnArgs.phases bit: no row pairs (one query row per item)
 SCHED_DEVICE = -1             # SasAttnArgs.num_fd: schedule summary read on the device
+QLENS_ARRAYS = 0              # sas_attention_launch_lens: q_prefix and act_q_lens arrays
+QLENS_CUMULATIVE = 1          # q_prefix is cu_seqlens_q
+QLENS_UNIFORM = 2             # total_tokens / batch rows each
 MERGE_SYNC_WORDS = 2 * AIC_CORE_NUM  # SasAttnArgs.merge_sync: uint64 arrival counters
 DEV_SCHED_MAX_BATCH = 4096
 DEV_SCHED_MAX_ITEMS = 16384
@@ -88,8 +91,9 @@ class SasAttnArgs(ctypes.Structure):
     ]
 
 
-EXPORTS = ("sas_metadata_build", "sas_metadata_build_device", "sas_workspace_bytes",
-           "sas_attention_launch", "sas_attention_launch_noalloc", "sas_kv_fp8_append",
+EXPORTS = ("sas_metadata_build", "sas_metadata_build_device", "sas_metadata_build_device_cu",
+           "sas_workspace_bytes", "sas_attention_launch", "sas_attention_launch_lens",
+           "sas_attention_launch_noalloc", "sas_merge_sync_take", "sas_kv_fp8_append",
            "sas_version", "sas_args_struct_size", "sas_last_error")
 NOALLOC_SCRATCH_BYTES = 72 << 20  # SAS_NOALLOC_SCRATCH_BYTES
 
@@ -117,10 +121,19 @@ def load() -> ctypes.CDLL:
         lib.sas_metadata_build_device.argtypes = ([ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p,
                                                    ctypes.c_int, ctypes.c_void_p] +
                                                   [ctypes.c_int] * 11 + [ctypes.c_void_p])
+        lib.sas_metadata_build_device_cu.restype = ctypes.c_int
+        lib.sas_metadata_build_device_cu.argtypes = ([ctypes.c_void_p, ctypes.c_int,
+                                                      ctypes.c_void_p, ctypes.c_void_p] +
+                                                     [ctypes.c_int] * 11 + [ctypes.c_void_p])
         lib.sas_workspace_bytes.restype = ctypes.c_int64
         lib.sas_workspace_bytes.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int]
         lib.sas_attention_launch.restype = ctypes.c_int
         lib.sas_attention_launch.argtypes = [ctypes.POINTER(SasAttnArgs), ctypes.c_void_p]
+        lib.sas_attention_launch_lens.restype = ctypes.c_int
+        lib.sas_attention_launch_lens.argtypes = [ctypes.POINTER(SasAttnArgs), ctypes.c_int,
+                                                  ctypes.c_void_p]
+        lib.sas_merge_sync_take.restype = ctypes.c_void_p
+        lib.sas_merge_sync_take.argtypes = [ctypes.c_void_p]
         lib.sas_attention_launch_noalloc.restype = ctypes.c_int
         lib.sas_attention_launch_noalloc.argtypes = [ctypes.POINTER(SasAttnArgs), ctypes.c_void_p]
         lib.sas_kv_fp8_append.restype = ctypes.c_int

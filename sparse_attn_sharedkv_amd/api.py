@@ -34,7 +34,7 @@ import torch
 
 from . import _lib
 from .metadata import (AIC_CORE_NUM, CFG_OFFSET, DEFAULT_CORE_NUM,  # noqa: F401
-                       DEFAULT_S2_BASE, FD_METADATA_SIZE, FD_OFFSET, SAS_META_SIZE,
+                       DEFAULT_MIN_SPLIT_BLOCKS, DEFAULT_S2_BASE, FD_METADATA_SIZE, FD_OFFSET, SAS_META_SIZE,
                        build_metadata, build_metadata_device, config_row, m_base_for,
                        m_base_valid)
 
@@ -73,6 +73,7 @@ class Prepared:
     layout_q: str = "TND"
     bsnd_shape: Optional[tuple] = None
     device: Optional[torch.device] = None
+    q_lens: int = _lib.QLENS_ARRAYS  # form of the query row counts (sas_attention_launch_lens)
     phase_bits: int = 0    # kernel-form bits every launch of this call carries (SAS_PHASE_FP8_QK)
     merge_in_kernel: bool = True  # split items merged by their last piece (SasAttnArgs.merge_sync)
 
@@ -138,19 +139,27 @@ def _schedule_buffer(dev: torch.device) -> torch.Tensor:
 
 # Arrival counters of the split-KV merge done inside the attention kernel
 # (SasAttnArgs.merge_sync): zero at rest, one buffer per (device, stream) so that
-# calls on different streams never share one; a call captured into a HIP graph
-# gets a buffer of its own (zeroed by a fill kernel recorded in the graph), kept
-# for the life of the process.
+# calls on different streams never share one. Calls captured into a HIP graph take
+# one of the library's own zeroed arrays (sas_merge_sync_take: one per capture and
+# stream, taken for the life of the process); when those are all taken, a buffer
+# zeroed by a fill kernel recorded in the graph.
 _MERGE_SYNC: dict = {}
 _CAPTURED_MERGE_SYNC: list = []
 
 
+def _captured_merge_sync(dev: torch.device, st: torch.cuda.Stream) -> int:
+    """Address of the counters for a call being captured on ``st``."""
+    with torch.cuda.device(dev):
+        at = _lib.load().sas_merge_sync_take(ctypes.c_void_p(st.cuda_stream))
+    if at:
+        return at
+    buf = torch.zeros(_lib.MERGE_SYNC_WORDS, dtype=torch.int64, device=dev)
+    with _DEVICE_SCHEDULES_LOCK:
+        _CAPTURED_MERGE_SYNC.append(buf)
+    return buf.data_ptr()
+
+
 def _merge_sync_buffer(dev: torch.device, st: torch.cuda.Stream) -> torch.Tensor:
-    if torch.cuda.is_current_stream_capturing():
-        buf = torch.zeros(_lib.MERGE_SYNC_WORDS, dtype=torch.int64, device=dev)
-        with _DEVICE_SCHEDULES_LOCK:
-            _CAPTURED_MERGE_SYNC.append(buf)
-        return buf
     key = (dev.index, st.cuda_stream)
     with _DEVICE_SCHEDULES_LOCK:
         buf = _MERGE_SYNC.get(key)
@@ -331,9 +340,23 @@ def prepare(q: torch.Tensor, *, ori_kv: torch.Tensor, cmp_kv: Optional[torch.Ten
     # ---- schedule (api.py:335-366) ----
     i32 = torch.int32
     seqused = seqused_kv.to(device=dev, dtype=i32).contiguous()
+    # Callers that launch right after preparing hand the kernels cu_seqlens_q itself,
+    # or nothing when every batch has as many rows, instead of arrays made from them
+    q_lens = _lib.QLENS_ARRAYS
+    act_q_d = cu_d = None
+    if _stream_schedule and nb > 0 and total > 0:
+        if layout_q == "TND":
+            q_lens = _lib.QLENS_CUMULATIVE
+            q_prefix = cu_d = cu_seqlens_q.to(device=dev, dtype=i32).reshape(-1).contiguous()
+            padded = False  # (the kernels zero the rows of no batch)
+        elif cu_seqlens_q is None:
+            q_lens = _lib.QLENS_UNIFORM
+            q_prefix = None
     if use_dev:
         # per-batch query rows and first flat token, computed on the GPU
-        if layout_q == "TND":
+        if q_lens != _lib.QLENS_ARRAYS:
+            pass
+        elif layout_q == "TND":
             cu_d = cu_seqlens_q.to(device=dev, dtype=i32).reshape(-1)
             act_q_d = (cu_d[1:] - cu_d[:-1]).contiguous()
             q_prefix = cu_d[:-1].contiguous()
@@ -346,7 +369,8 @@ def prepare(q: torch.Tensor, *, ori_kv: torch.Tensor, cmp_kv: Optional[torch.Ten
                 act_q_d = torch.full((nb,), total // max(nb, 1), dtype=i32, device=dev)
         if metadata is None:
             metadata_dev = build_metadata_device(
-                batch=nb, act_q=act_q_d, act_kv=seqused, num_heads=int(n1),
+                batch=nb, act_q=act_q_d, cu_q=cu_d if act_q_d is None else None,
+                uniform_q=total // max(nb, 1), act_kv=seqused, num_heads=int(n1),
                 ori_win_left=int(ori_win_left), scenario=scenario, cmp_ratio=cmp_ratio_eff,
                 cmp_topk=int(k), core_num=int(core_num),
                 out=_schedule_buffer(dev) if _stream_schedule else None, item64=item64,
@@ -362,9 +386,17 @@ def prepare(q: torch.Tensor, *, ori_kv: torch.Tensor, cmp_kv: Optional[torch.Ten
         cfg = dict(num_fa=cap, num_fd=_lib.SCHED_DEVICE, num_partial_slots=2 * cap,
                    s2_base=DEFAULT_S2_BASE, m_base=m_base)
         # pieces per item are not known on the host: expect at most two when the
-        # items are at least half as many as the workgroups
+        # items are at least half as many as the workgroups, or when the longest
+        # possible list has too few blocks for more
         items = total * ((n1 + cfg["m_base"] - 1) // cfg["m_base"])
-        few_pieces = int(core_num) <= MERGE_IN_KERNEL_MAX_PIECES * items
+        longest = int(ori_win_left) + 1
+        if scenario == 3:
+            longest += int(k)
+        elif scenario == 2:
+            longest += cmp_block_table.shape[1] * cmp_kv.shape[1]
+        most = -(-longest // DEFAULT_S2_BASE) // DEFAULT_MIN_SPLIT_BLOCKS
+        few_pieces = (int(core_num) <= MERGE_IN_KERNEL_MAX_PIECES * items
+                      or most <= MERGE_IN_KERNEL_MAX_PIECES)
     elif metadata is None:
         kv_host = tuple(int(x) for x in seqused_kv.to(torch.int32).cpu().tolist())
         md, max_pieces = _cached_schedule(tuple(act_q), kv_host, int(n1), int(ori_win_left),
@@ -389,7 +421,7 @@ def prepare(q: torch.Tensor, *, ori_kv: torch.Tensor, cmp_kv: Optional[torch.Ten
     cmp_kv_d = cmp_kv.contiguous() if cmp_kv is not None else None
     cmp_bt = cmp_block_table.to(device=dev, dtype=i32).contiguous() if cmp_kv is not None else None
     idx_d = idx_flat.to(device=dev, dtype=i32).contiguous() if idx_flat is not None else None
-    if not use_dev:
+    if not use_dev and q_lens == _lib.QLENS_ARRAYS:
         q_prefix = torch.tensor(prefix, dtype=i32).to(dev, non_blocking=True)
         act_q_d = torch.tensor(act_q, dtype=i32).to(dev, non_blocking=True)
     sinks_d = sinks.to(device=dev, dtype=torch.float32).contiguous()
@@ -431,7 +463,7 @@ def prepare(q: torch.Tensor, *, ori_kv: torch.Tensor, cmp_kv: Optional[torch.Ten
             sinks_d, metadata_dev, out, lse, ws]
     return Prepared(args=a, keep=keep, out=out, lse=lse, layout_q=layout_q,
                     bsnd_shape=None if layout_q == "TND" else (nb, total // max(nb, 1), n1, dv),
-                    device=dev, phase_bits=(_lib.SAS_PHASE_FP8_QK if fp8_qk else 0) |
+                    device=dev, q_lens=q_lens, phase_bits=(_lib.SAS_PHASE_FP8_QK if fp8_qk else 0) |
                     (_lib.SAS_PHASE_PIPELINED if _pipelined else 0) |
                     (_lib.SAS_PHASE_ROW_ITEMS if _row_items else 0),
                     merge_in_kernel=few_pieces if _separate_merge is None
@@ -458,14 +490,17 @@ def launch(prep: Prepared, stream: Optional[torch.cuda.Stream] = None, phases: i
     lib = _lib.load()
     st = stream if stream is not None else torch.cuda.current_stream(prep.device)
     prep.args.phases = int(phases) | prep.phase_bits
-    if prep.merge_in_kernel and prep.args.workspace:
+    if not (prep.merge_in_kernel and prep.args.workspace):
+        prep.args.merge_sync = None
+    elif torch.cuda.is_current_stream_capturing():
+        prep.args.merge_sync = _captured_merge_sync(prep.device, st)
+    else:
         sync = _merge_sync_buffer(prep.device, st)
         prep.args.merge_sync = sync.data_ptr()
         if not any(t is sync for t in prep.keep):
             prep.keep.append(sync)
-    else:
-        prep.args.merge_sync = None
-    rc = lib.sas_attention_launch(ctypes.byref(prep.args), ctypes.c_void_p(st.cuda_stream))
+    rc = lib.sas_attention_launch_lens(ctypes.byref(prep.args), prep.q_lens,
+                                       ctypes.c_void_p(st.cuda_stream))
     if rc != _lib.SAS_OK:
         raise RuntimeError(_lib.last_error())
 

@@ -183,6 +183,43 @@ __device__ inline int32_t ld_uniform(const int32_t* p) {
   return *(const __attribute__((address_space(4))) int32_t*)p;
 }
 
+// Query rows of the batches, in one of three forms (SAS_QLENS_*, told apart by the
+// null pointers the launch leaves): `first` and `rows` arrays; cumulative row counts
+// (first only: batch b's rows end where those of b + 1 begin); or as many rows in
+// every batch (neither). Batch b starts at token start(first[b]) and has
+// count(rows[b], first[b]) rows; reads of the unused arrays go to seqused_kv.
+struct QRows {
+  const int32_t *first, *rows;
+  int uniform;      // rows of every batch, or -1
+  bool cumulative;
+  __device__ explicit QRows(const SasAttnArgs& a)
+      : first(a.q_prefix ? a.q_prefix : a.seqused_kv),
+        rows(!a.q_prefix ? a.seqused_kv : a.act_q_lens ? a.act_q_lens : a.q_prefix + 1),
+        uniform(a.q_prefix ? -1 : a.total_tokens / a.batch),
+        cumulative(a.q_prefix && !a.act_q_lens) {}
+  __device__ int start(int b, int first_b) const { return uniform < 0 ? first_b : b * uniform; }
+  __device__ int count(int rows_b, int first_b) const {
+    return uniform >= 0 ? uniform : cumulative ? rows_b - first_b : rows_b;
+  }
+};
+
+// Cumulative row counts: tokens outside [lo, hi) belong to no row of the schedule;
+// their output and lse rows are zeroed, spread over the workgroups in use (a fill of
+// every output row in front of the kernel took 12 us of a 128 x 128-head decode call).
+template <typename T>
+__device__ inline void zero_unowned_rows(const SasAttnArgs& a, int lo, int hi, int wg, int nwg,
+                                         int tid, int nthreads) {
+  lo = lo < 0 ? 0 : (lo < a.total_tokens ? lo : a.total_tokens);
+  hi = hi < lo ? lo : (hi < a.total_tokens ? hi : a.total_tokens);
+  const int n = lo + a.total_tokens - hi;
+  for (int r = wg; r < n; r += nwg) {
+    const size_t row = (size_t)(r < lo ? r : hi + r - lo) * a.num_heads;
+    i32x4* out = (i32x4*)((T*)a.out + row * a.head_dim_v);
+    for (int k = tid; k < a.num_heads * a.head_dim_v / 8; k += nthreads) out[k] = (i32x4){0, 0, 0, 0};
+    for (int k = tid; k < a.num_heads; k += nthreads) a.lse[row + k] = 0.0f;
+  }
+}
+
 template <int N>
 __device__ inline void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -622,6 +659,10 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
   if (fa_row >= nfa || (int)(blockIdx.x >> 3) >= per_xcd) return;
   const int32_t* fa = a.metadata + fa_row * SAS_FA_METADATA_SIZE;
   if (fa[0] == 0) return;
+  // where the whole schedule ends (loaded beside this row's cursors)
+  const int32_t* fa_last = a.metadata + (nfa - 1) * SAS_FA_METADATA_SIZE;
+  const int last_b = fa_last[4] < a.batch ? fa_last[4] : a.batch;
+  const int last_m = fa_last[4] < a.batch ? fa_last[5] : 0;
   int b = fa[1], m = fa[2];
   const int j_start = fa[3];
   const int b_end = fa[4], s_end = fa[5], j_end = fa[6];
@@ -639,13 +680,14 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
   // With at most 64 batches, every batch's lengths and query offset sit in one
   // lane each, loaded at the start beside the metadata row (they no longer wait
   // for it: the item's batch picks its lane).
+  const QRows qrows(a);
   const bool lens_in_lanes = a.batch <= 64;
   int lane_aq = 0, lane_kv = 0, lane_qp = 0;
   if (lens_in_lanes) {
     const int lb = lane < a.batch ? lane : a.batch - 1;
-    lane_aq = a.act_q_lens[lb];
+    lane_aq = qrows.rows[lb];
     lane_kv = a.seqused_kv[lb];
-    lane_qp = a.q_prefix[lb];
+    lane_qp = qrows.first[lb];
   }
   if (tid < 2) first_neg[tid] = INT32_MAX;
   // piece index of the first item when it continues a split item
@@ -662,7 +704,15 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
   // the lane-held lengths are waited for here, once: read first inside the item
   // loop, whose later iterations have output stores and query loads in flight,
   // they would make the head of every item wait for those
-  asm volatile("" ::"v"(lane_aq), "v"(lane_kv), "v"(lane_qp));
+  lane_aq = qrows.count(lane_aq, lane_qp);
+  lane_qp = qrows.start(lane, lane_qp);
+  asm volatile("" : "+v"(lane_aq), "+v"(lane_kv), "+v"(lane_qp));
+  // cumulative row counts: the tokens [tok_lo, tok_hi) of the schedule's rows
+  int tok_lo = 0, tok_hi = a.total_tokens;
+  if (qrows.cumulative) {
+    tok_lo = ld_uniform(qrows.first);
+    tok_hi = ld_uniform(qrows.first + last_b) + last_m / ((a.num_heads + MB - 1) / MB);
+  }
   int item_par = 0;  // which first_neg slot the next top-k scan uses
   bool first_item = true;
   // query fragment of this wave's dims half (B operand of Sᵀ = K·Qᵀ); the next
@@ -678,9 +728,10 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
       akv = __builtin_amdgcn_readlane(lane_kv, bc);
       qp = __builtin_amdgcn_readlane(lane_qp, bc);
     } else {
-      aq = ld_uniform(a.act_q_lens + bc);
+      const int first_b = ld_uniform(qrows.first + bc);
+      aq = qrows.count(ld_uniform(qrows.rows + bc), first_b);
       akv = ld_uniform(a.seqused_kv + bc);
-      qp = ld_uniform(a.q_prefix + bc);
+      qp = qrows.start(bc, first_b);
     }
   };
   // this wave's query fragment of (token, head), zero for rows out of range
@@ -1326,6 +1377,7 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
     first_item = false;
     ++m;
   }
+  zero_unowned_rows<T>(a, tok_lo, tok_hi, fa_row, nfa, tid, NT);
 }
 
 // ---------------------------------------------------------------------------
@@ -1496,6 +1548,10 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
   if (fa_row >= nfa || (int)(blockIdx.x >> 3) >= per_xcd) return;
   const int32_t* fa = a.metadata + fa_row * SAS_FA_METADATA_SIZE;
   if (fa[0] == 0) return;
+  // where the whole schedule ends (loaded beside this row's cursors)
+  const int32_t* fa_last = a.metadata + (nfa - 1) * SAS_FA_METADATA_SIZE;
+  const int last_b = fa_last[4] < a.batch ? fa_last[4] : a.batch;
+  const int last_m = fa_last[4] < a.batch ? fa_last[5] : 0;
   int b = fa[1], m = fa[2];
   const int j_start = fa[3];
   const int b_end = fa[4], s_end = fa[5], j_end = fa[6];
@@ -1507,6 +1563,14 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
   const float sc = a.softmax_scale * LOG2E;
   if (tid < 2) first_neg[tid] = INT32_MAX;
   __syncthreads();
+
+  const QRows qrows(a);
+  // cumulative row counts: the tokens [tok_lo, tok_hi) of the schedule's rows
+  int tok_lo = 0, tok_hi = a.total_tokens;
+  if (qrows.cumulative) {
+    tok_lo = ld_uniform(qrows.first);
+    tok_hi = ld_uniform(qrows.first + last_b) + last_m / ((a.num_heads + MB - 1) / MB);
+  }
 
   // Sinks of this lane's softmax head in the (at most two) head blocks of an
   // item, loaded once: a load per item would also wait for the previous item's
@@ -1524,9 +1588,10 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
     int act_q, act_kv, qpre;
     auto load_batch = [&] {
       const int bc = b < a.batch ? b : a.batch - 1;
-      act_q = ld_uniform(a.act_q_lens + bc);
+      const int first_b = ld_uniform(qrows.first + bc);
+      act_q = qrows.count(ld_uniform(qrows.rows + bc), first_b);
       act_kv = ld_uniform(a.seqused_kv + bc);
-      qpre = ld_uniform(a.q_prefix + bc);
+      qpre = qrows.start(bc, first_b);
     };
     load_batch();
     // normalise the cursor: skip batches with no (more) query rows
@@ -2248,6 +2313,7 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
     first_item = false;
     ++m;
   }
+  zero_unowned_rows<T>(a, tok_lo, tok_hi, fa_row, nfa, tid, NT);
 }
 
 }  // namespace sas
@@ -2311,7 +2377,8 @@ __device__ __forceinline__ void merge_task(const SasAttnArgs& a, int task) {
   const int h = (m - s * hblocks) * mb + hloc;  // query head
   const bool store = g0 + hh < hn && h < a.num_heads;
   const float sink = a.sinks[h < a.num_heads ? h : a.num_heads - 1];
-  const int tok = a.q_prefix[b] + s;
+  const QRows qrows(a);
+  const int tok = qrows.start(b, qrows.first[b]) + s;
   // lse = log(e^sink + Σ_i e^lse_i); weights e^(lse_i - lse); the sums keep the
   // piece order 0, 1, 2, ...
   f32x4 o[PER];
@@ -2529,16 +2596,35 @@ static hipError_t dispatch_fp8(const SasAttnArgs& a, hipStream_t st) {
 }  // namespace sas
 
 extern "C" int sas_attention_launch(const SasAttnArgs* a, void* stream) {
+  return sas_attention_launch_lens(a, SAS_QLENS_ARRAYS, stream);
+}
+
+extern "C" int sas_attention_launch_lens(const SasAttnArgs* args, int q_lens, void* stream) {
   using sas::set_error;
-  if (!a) {
+  if (!args) {
     set_error("sas_attention_launch: null args");
     return SAS_E_INVALID;
   }
-  if (!a->q || !a->ori_kv || !a->ori_block_table || !a->q_prefix || !a->act_q_lens ||
-      !a->seqused_kv || !a->sinks || !a->metadata || !a->out || !a->lse) {
+  if (q_lens < SAS_QLENS_ARRAYS || q_lens > SAS_QLENS_UNIFORM) {
+    set_error("sas_attention_launch_lens: unknown form of the query row counts");
+    return SAS_E_INVALID;
+  }
+  if (!args->q || !args->ori_kv || !args->ori_block_table ||
+      (q_lens != SAS_QLENS_UNIFORM && !args->q_prefix) ||
+      (q_lens == SAS_QLENS_ARRAYS && !args->act_q_lens) ||
+      !args->seqused_kv || !args->sinks || !args->metadata || !args->out || !args->lse) {
     set_error("sas_attention_launch: null tensor pointer");
     return SAS_E_INVALID;
   }
+  if (q_lens == SAS_QLENS_UNIFORM && args->batch > 0 && args->total_tokens % args->batch != 0) {
+    set_error("sas_attention_launch_lens: total_tokens must be a multiple of batch");
+    return SAS_E_INVALID;
+  }
+  // the kernels tell the forms apart by the null pointers (QRows)
+  SasAttnArgs form = *args;
+  if (q_lens != SAS_QLENS_ARRAYS) form.act_q_lens = nullptr;
+  if (q_lens == SAS_QLENS_UNIFORM) form.q_prefix = nullptr;
+  const SasAttnArgs* const a = &form;
   if (a->head_dim != 512 && a->head_dim != 576) {
     set_error("sas_attention_launch: head_dim must be 512 or 576");
     return SAS_E_UNSUPPORTED;
@@ -2689,7 +2775,58 @@ extern "C" int sas_attention_launch_noalloc(const SasAttnArgs* a, void* stream) 
   return sas_attention_launch(&b, stream);
 }
 
-extern "C" int sas_version(void) { return 114; }
+// ---------------------------------------------------------------------------
+// Arrival counters for captured calls
+// ---------------------------------------------------------------------------
+namespace sas {
+// Zero when the code object is loaded and zero again after every call that used
+// them, so a graph that owns an array needs no fill in front of its kernels (a
+// fill of 8 KB delayed each replay's attention by about 4.5 us).
+__device__ unsigned long long g_sync_pool[SAS_MERGE_SYNC_POOL][SAS_MERGE_SYNC_WORDS];
+struct SyncPool {
+  char* base = nullptr;
+  int used = 0;
+  unsigned long long capture = 0;  // the capture and stream that took the last array
+  hipStream_t stream = nullptr;
+};
+static SyncPool g_sync[MAX_DEVICES];
+static std::mutex g_sync_mu;
+}  // namespace sas
+
+extern "C" uint64_t* sas_merge_sync_take(void* stream) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= sas::MAX_DEVICES) return nullptr;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long capture = 0;
+  if (hipStreamGetCaptureInfo((hipStream_t)stream, &status, &capture) != hipSuccess ||
+      status != hipStreamCaptureStatusActive) {
+    sas::set_error("sas_merge_sync_take: the stream is not capturing");
+    return nullptr;
+  }
+  std::lock_guard<std::mutex> lock(sas::g_sync_mu);
+  sas::SyncPool& p = sas::g_sync[dev];
+  if (!p.base) {
+    void* at = nullptr;
+    if (hipGetSymbolAddress(&at, HIP_SYMBOL(sas::g_sync_pool)) != hipSuccess || !at) {
+      sas::set_error("sas_merge_sync_take: hipGetSymbolAddress failed");
+      return nullptr;
+    }
+    p.base = (char*)at;
+  }
+  // calls of one capture on one stream run one after another: they share an array
+  if (p.used == 0 || p.capture != capture || p.stream != (hipStream_t)stream) {
+    if (p.used == SAS_MERGE_SYNC_POOL) {
+      sas::set_error("sas_merge_sync_take: every array is taken");
+      return nullptr;
+    }
+    ++p.used;
+    p.capture = capture;
+    p.stream = (hipStream_t)stream;
+  }
+  return (uint64_t*)(p.base + (size_t)(p.used - 1) * SAS_MERGE_SYNC_WORDS * 8);
+}
+
+extern "C" int sas_version(void) { return 115; }
 
 extern "C" int sas_args_struct_size(void) { return (int)sizeof(SasAttnArgs); }
 

@@ -178,6 +178,10 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
   if (fa_row >= nfa || (int)(blockIdx.x >> 3) >= per_xcd) return;
   const int32_t* fa = a.metadata + fa_row * SAS_FA_METADATA_SIZE;
   if (fa[0] == 0) return;
+  // where the whole schedule ends (loaded beside this row's cursors)
+  const int32_t* fa_last = a.metadata + (nfa - 1) * SAS_FA_METADATA_SIZE;
+  const int last_b = fa_last[4] < a.batch ? fa_last[4] : a.batch;
+  const int last_m = fa_last[4] < a.batch ? fa_last[5] : 0;
   int b = fa[1], m = fa[2];
   const int j_start = fa[3];
   const int b_end = fa[4], s_end = fa[5], j_end = fa[6];
@@ -195,13 +199,14 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
   // With at most 64 batches, every batch's lengths and query offset sit in one
   // lane each, loaded at the start beside the metadata row; otherwise they are
   // scalar loads per item.
+  const QRows qrows(a);
   const bool lens_in_lanes = a.batch <= 64;
   int lane_aq = 0, lane_kv = 0, lane_qp = 0;
   if (lens_in_lanes) {
     const int lb = lane < a.batch ? lane : a.batch - 1;
-    lane_aq = a.act_q_lens[lb];
+    lane_aq = qrows.rows[lb];
     lane_kv = a.seqused_kv[lb];
-    lane_qp = a.q_prefix[lb];
+    lane_qp = qrows.first[lb];
   }
   if (tid < 2) first_neg[tid] = INT32_MAX;
   // piece index of the first item when it continues a split item
@@ -209,7 +214,15 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
   __syncthreads();
   // sink of this lane's head (an item holds every head: one head block)
   const float sink_h = hlocal < a.num_heads ? a.sinks[hlocal] : -INFINITY;
-  asm volatile("" ::"v"(lane_aq), "v"(lane_kv), "v"(lane_qp));
+  lane_aq = qrows.count(lane_aq, lane_qp);
+  lane_qp = qrows.start(lane, lane_qp);
+  asm volatile("" : "+v"(lane_aq), "+v"(lane_kv), "+v"(lane_qp));
+  // cumulative row counts: the tokens [tok_lo, tok_hi) of the schedule's rows
+  int tok_lo = 0, tok_hi = a.total_tokens;
+  if (qrows.cumulative) {
+    tok_lo = ld_uniform(qrows.first);
+    tok_hi = ld_uniform(qrows.first + last_b) + last_m / ((a.num_heads + IMB - 1) / IMB);
+  }
   int item_par = 0;  // which first_neg slot the next top-k scan uses
   bool first_item = true;
   const int hblocks = (a.num_heads + IMB - 1) / IMB;
@@ -220,9 +233,10 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
       akv = __builtin_amdgcn_readlane(lane_kv, bc);
       qp = __builtin_amdgcn_readlane(lane_qp, bc);
     } else {
-      aq = ld_uniform(a.act_q_lens + bc);
+      const int first_b = ld_uniform(qrows.first + bc);
+      aq = qrows.count(ld_uniform(qrows.rows + bc), first_b);
       akv = ld_uniform(a.seqused_kv + bc);
-      qp = ld_uniform(a.q_prefix + bc);
+      qp = qrows.start(bc, first_b);
     }
   };
   for (;;) {
@@ -1009,6 +1023,7 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
     if (pair) ++m;
     ++m;
   }
+  zero_unowned_rows<T>(a, tok_lo, tok_hi, fa_row, nfa, tid, NT);
 }
 
 }  // namespace sas

@@ -271,6 +271,7 @@ __device__ int64_t block_excl_scan(int64_t v, int64_t* wsum, int64_t* total) {
 struct Params {
   int32_t* meta;
   const int32_t* act_q;         // [batch] query rows, or null: every batch has uniform_q
+  const int32_t* cu_q;          // or [batch + 1] cumulative query rows
   const int32_t* seqused_kv;    // [batch]
   int32_t batch, uniform_q, num_heads, m_base, ori_win_left, scenario, cmp_ratio, cmp_topk;
   int32_t num_cores, s2_base, min_split_blocks, fd_head_chunk;
@@ -306,7 +307,9 @@ __global__ __launch_bounds__(NT) void sched_kernel(const Params p) {
 
   const int batch = p.batch;
   const int hblocks = (p.num_heads + p.m_base - 1) / p.m_base;
-  auto rows_of = [&](int b) { return p.act_q ? p.act_q[b] : p.uniform_q; };
+  auto rows_of = [&](int b) {
+    return p.cu_q ? p.cu_q[b + 1] - p.cu_q[b] : p.act_q ? p.act_q[b] : p.uniform_q;
+  };
   // ---- first item of every batch: thread t owns batches BPT t .. BPT t + BPT - 1 ----
   {
     int64_t cnt[BPT];
@@ -636,14 +639,13 @@ __global__ __launch_bounds__(NT) void sched_kernel(const Params p) {
 
 }  // namespace sasdev
 
-extern "C" int sas_metadata_build_device(int32_t* meta, int batch, const int32_t* act_q,
-                                         int uniform_q, const int32_t* seqused_kv, int num_heads,
-                                         int m_base, int ori_win_left, int scenario, int cmp_ratio,
-                                         int cmp_topk, int num_cores, int s2_base,
-                                         int min_split_blocks, int fd_head_chunk, int reuse,
-                                         void* stream) {
+static int build_device(int32_t* meta, int batch, const int32_t* act_q, const int32_t* cu_q,
+                        int uniform_q, const int32_t* seqused_kv, int num_heads, int m_base,
+                        int ori_win_left, int scenario, int cmp_ratio, int cmp_topk, int num_cores,
+                        int s2_base, int min_split_blocks, int fd_head_chunk, int reuse,
+                        void* stream) {
   if (!meta || batch < 0 || batch > SAS_DEV_SCHED_MAX_BATCH || (batch > 0 && !seqused_kv) ||
-      (!act_q && uniform_q < 0)) {
+      (!act_q && !cu_q && uniform_q < 0)) {
     sas::set_error("sas_metadata_build_device: null pointer or batch out of range");
     return SAS_E_INVALID;
   }
@@ -657,6 +659,7 @@ extern "C" int sas_metadata_build_device(int32_t* meta, int batch, const int32_t
   sasdev::Params p;
   p.meta = meta;
   p.act_q = act_q;
+  p.cu_q = cu_q;
   p.seqused_kv = seqused_kv;
   p.batch = batch;
   p.uniform_q = uniform_q;
@@ -678,4 +681,26 @@ extern "C" int sas_metadata_build_device(int32_t* meta, int batch, const int32_t
     return SAS_E_HIP;
   }
   return SAS_OK;
+}
+
+extern "C" int sas_metadata_build_device(int32_t* meta, int batch, const int32_t* act_q,
+                                         int uniform_q, const int32_t* seqused_kv, int num_heads,
+                                         int m_base, int ori_win_left, int scenario, int cmp_ratio,
+                                         int cmp_topk, int num_cores, int s2_base,
+                                         int min_split_blocks, int fd_head_chunk, int reuse,
+                                         void* stream) {
+  return build_device(meta, batch, act_q, nullptr, uniform_q, seqused_kv, num_heads, m_base,
+                      ori_win_left, scenario, cmp_ratio, cmp_topk, num_cores, s2_base,
+                      min_split_blocks, fd_head_chunk, reuse, stream);
+}
+
+extern "C" int sas_metadata_build_device_cu(int32_t* meta, int batch, const int32_t* cu_q,
+                                            const int32_t* seqused_kv, int num_heads, int m_base,
+                                            int ori_win_left, int scenario, int cmp_ratio,
+                                            int cmp_topk, int num_cores, int s2_base,
+                                            int min_split_blocks, int fd_head_chunk, int reuse,
+                                            void* stream) {
+  return build_device(meta, batch, nullptr, cu_q, -1, seqused_kv, num_heads, m_base, ori_win_left,
+                      scenario, cmp_ratio, cmp_topk, num_cores, s2_base, min_split_blocks,
+                      fd_head_chunk, reuse, stream);
 }

@@ -170,9 +170,9 @@ def build_metadata(*, act_q: Sequence[int], act_kv: Sequence[int], num_heads: in
 def device_lengths(*, layout_q: str, layout_kv: str, device, cu_seqlens_q=None,
                    cu_seqlens_ori_kv=None, seqused_q=None, seqused_kv=None, batch_size: int = 0,
                    max_seqlen_q: int = 0, max_seqlen_kv: int = 0):
-    """``resolve_lengths`` on the GPU: ``(batch, act_q, uniform_q, act_kv)`` with int32
-    device tensors (``act_q`` is None when every batch has ``uniform_q`` rows). Only
-    tensor shapes are read on the host."""
+    """``resolve_lengths`` on the GPU: ``(batch, act_q, cu_q, uniform_q, act_kv)`` with int32
+    device tensors: the query rows are ``act_q``, or the differences of ``cu_q``, or
+    ``uniform_q`` in every batch. Only tensor shapes are read on the host."""
     i32 = torch.int32
 
     def dev(t):
@@ -187,12 +187,12 @@ def device_lengths(*, layout_q: str, layout_kv: str, device, cu_seqlens_q=None,
         batch = torch.as_tensor(cu_seqlens_q).numel() - 1
     else:
         batch = int(batch_size)
-    act_q, uniform_q = None, 0
+    act_q = cu_q = None
+    uniform_q = 0
     if nonempty(seqused_q):
         act_q = dev(seqused_q)[:batch].contiguous()
     elif layout_q == "TND" and nonempty(cu_seqlens_q):
-        c = dev(cu_seqlens_q)
-        act_q = (c[1:batch + 1] - c[:batch]).contiguous()
+        cu_q = dev(cu_seqlens_q).contiguous()
     else:
         uniform_q = int(max_seqlen_q)
     if nonempty(seqused_kv):
@@ -202,12 +202,13 @@ def device_lengths(*, layout_q: str, layout_kv: str, device, cu_seqlens_q=None,
         act_kv = (c[1:batch + 1] - c[:batch]).contiguous()
     else:
         act_kv = torch.full((batch,), int(max_seqlen_kv), dtype=i32, device=device)
-    return batch, act_q, uniform_q, act_kv
+    return batch, act_q, cu_q, uniform_q, act_kv
 
 
 def build_metadata_device(*, batch: int, act_q: Optional[torch.Tensor], act_kv: torch.Tensor,
                           num_heads: int, ori_win_left: int, scenario: int, cmp_ratio: int,
-                          cmp_topk: int, uniform_q: int = 0, core_num: int = DEFAULT_CORE_NUM,
+                          cmp_topk: int, uniform_q: int = 0,
+                          cu_q: Optional[torch.Tensor] = None, core_num: int = DEFAULT_CORE_NUM,
                           s2_base: int = DEFAULT_S2_BASE,
                           min_split_blocks: int = DEFAULT_MIN_SPLIT_BLOCKS,
                           fd_head_chunk: int = DEFAULT_FD_HEAD_CHUNK,
@@ -216,8 +217,9 @@ def build_metadata_device(*, batch: int, act_q: Optional[torch.Tensor], act_kv: 
                           m_base: Optional[int] = None, fp8_rows: bool = False) -> torch.Tensor:
     """Run the on-device scheduler (``sas_metadata_build_device``) on the current stream.
 
-    ``act_q`` / ``act_kv``: int32 ``[batch]`` tensors on the GPU (``act_q`` None: every
-    batch has ``uniform_q`` query rows). Returns the int32 ``SAS_META_SIZE`` schedule on
+    ``act_q`` / ``act_kv``: int32 ``[batch]`` tensors on the GPU (``act_q`` None: the query
+    rows are the differences of ``cu_q``, int32 ``[batch + 1]``, or ``uniform_q`` in every
+    batch). Returns the int32 ``SAS_META_SIZE`` schedule on
     the same GPU, word for word what ``build_metadata`` returns for the same lengths;
     nothing is read back. Lengths the host cannot check (negative, too many items) leave
     a schedule the attention launch turns into NaN outputs.
@@ -237,6 +239,11 @@ def build_metadata_device(*, batch: int, act_q: Optional[torch.Tensor], act_kv: 
         if t is not None and (t.dtype != torch.int32 or t.device != dev or t.numel() < batch
                               or not t.is_contiguous()):
             raise ValueError("act_q / act_kv must be contiguous int32 [batch] tensors on one GPU")
+    if act_q is not None:
+        cu_q = None
+    if cu_q is not None and (cu_q.dtype != torch.int32 or cu_q.device != dev
+                             or cu_q.numel() < batch + 1 or not cu_q.is_contiguous()):
+        raise ValueError("cu_q must be a contiguous int32 [batch + 1] tensor on the same GPU")
     reuse = out is not None
     if out is None:
         out = torch.empty(SAS_META_SIZE, dtype=torch.int32, device=dev)
@@ -246,13 +253,18 @@ def build_metadata_device(*, batch: int, act_q: Optional[torch.Tensor], act_kv: 
     st = stream if stream is not None else torch.cuda.current_stream(dev)
     if m_base is None:
         m_base = m_base_for(int(num_heads), item64, int(batch), fp8_rows)
-    rc = lib.sas_metadata_build_device(
-        ctypes.c_void_p(out.data_ptr()), int(batch),
-        ctypes.c_void_p(act_q.data_ptr() if act_q is not None else 0), int(uniform_q),
-        ctypes.c_void_p(act_kv.data_ptr()), int(num_heads), int(m_base),
-        int(ori_win_left), int(scenario), int(cmp_ratio), int(cmp_topk), int(core_num),
-        int(s2_base), int(min_split_blocks), int(fd_head_chunk), int(reuse),
-        ctypes.c_void_p(st.cuda_stream))
+    common = (ctypes.c_void_p(act_kv.data_ptr()), int(num_heads), int(m_base),
+              int(ori_win_left), int(scenario), int(cmp_ratio), int(cmp_topk), int(core_num),
+              int(s2_base), int(min_split_blocks), int(fd_head_chunk), int(reuse),
+              ctypes.c_void_p(st.cuda_stream))
+    if cu_q is not None:
+        rc = lib.sas_metadata_build_device_cu(ctypes.c_void_p(out.data_ptr()), int(batch),
+                                              ctypes.c_void_p(cu_q.data_ptr()), *common)
+    else:
+        rc = lib.sas_metadata_build_device(
+            ctypes.c_void_p(out.data_ptr()), int(batch),
+            ctypes.c_void_p(act_q.data_ptr() if act_q is not None else 0), int(uniform_q),
+            *common)
     if rc < 0:
         raise ValueError(_lib.last_error())
     return out
@@ -338,12 +350,12 @@ def sparse_attn_sharedkv_metadata(
     fp8_rows = _is_fp8(kv_cache_dtype)
     if device is not None and torch.device(device).type == "cuda":
         # scheduled on that GPU from device-resident lengths: nothing is read back
-        batch, act_q, uniform_q, act_kv = device_lengths(
+        batch, act_q, cu_q, uniform_q, act_kv = device_lengths(
             layout_q=layout_q, layout_kv=layout_kv, device=device, cu_seqlens_q=cu_seqlens_q,
             cu_seqlens_ori_kv=cu_seqlens_ori_kv, seqused_q=seqused_q, seqused_kv=seqused_kv,
             batch_size=batch_size, max_seqlen_q=max_seqlen_q, max_seqlen_kv=max_seqlen_kv)
-        return build_metadata_device(batch=batch, act_q=act_q, uniform_q=uniform_q,
-                                     act_kv=act_kv, num_heads=num_heads_q,
+        return build_metadata_device(batch=batch, act_q=act_q, cu_q=cu_q,
+                                     uniform_q=uniform_q, act_kv=act_kv, num_heads=num_heads_q,
                                      ori_win_left=ori_win_left, scenario=scenario,
                                      cmp_ratio=max(int(cmp_ratio), 1), cmp_topk=int(cmp_topk),
                                      core_num=core_num, item64=item64, fp8_rows=fp8_rows)
