@@ -271,6 +271,237 @@ __device__ inline void gather_dwords_wait(int (&v)[N], const int32_t* const (&p)
 // unwritten pool row need not be. Large enough for every row format.
 __device__ __attribute__((aligned(256))) unsigned char g_zero_row[1152];
 
+// What the attention kernels are launched with: the call's arguments and the
+// divisors of the index arithmetic as multipliers.
+struct FastDiv {
+  uint32_t mul, shift;
+  // floor(n / d), 0 <= n < 2^31: with l = ceil(log2 d) and mul = ceil(2^(31 + l) / d),
+  // mul * d exceeds 2^(31 + l) by less than d <= 2^l, so n times the excess stays
+  // below 2^(31 + l) and the quotient exact
+  static FastDiv of(int d) {
+    uint32_t l = 0;
+    while (((int64_t)1 << l) < d) ++l;
+    return {(uint32_t)((((uint64_t)1 << (31 + l)) + (uint64_t)d - 1) / (uint64_t)d), l};
+  }
+  __device__ int div(int n) const { return (int)(__umulhi((uint32_t)n << 1, mul) >> shift); }
+};
+struct KernelArgs : SasAttnArgs {
+  FastDiv ori_bs, cmp_bs, ratio;  // of the block sizes and cmp_ratio
+};
+
+// The launch's arguments, read again from the kernel argument segment. Each phase of an
+// item (its geometry and rows, the epilogue, the merge) takes its own copy: the few
+// scalar loads it needs hit the scalar cache, while arguments (and what the compiler
+// derives from them outside the item loop) kept in registers across the tile loop
+// overflow the scalar registers into lanes of vector registers, and that spilling
+// alone was a third of the instructions before a call's first row loads.
+__device__ __forceinline__ KernelArgs fresh_args() {
+  typedef const __attribute__((address_space(4))) uint32_t* seg_p;
+  seg_p p = (seg_p)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  KernelArgs a;
+  static_assert(sizeof(KernelArgs) % 4 == 0, "whole words");
+  uint32_t words[sizeof(KernelArgs) / 4];
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(KernelArgs) / 4); ++i) words[i] = p[i];
+  __builtin_memcpy(&a, words, sizeof(a));
+  return a;
+}
+
+// item_geom (sas_items.h) of one item with the division by cmp_ratio as a product: an
+// item's last position + 1 never exceeds its length, so one at or below 0 is an item
+// that attends nothing.
+__device__ inline ItemGeom item_geom_at(const KernelArgs& a, int act_q, int act_kv, int s) {
+  const int64_t end64 = (int64_t)act_kv - act_q + s + 1;
+  const int end = end64 < 0 ? 0 : (end64 > INT32_MAX ? INT32_MAX : (int)end64);
+  ItemGeom g = {0, 0, 0, 0};
+  if (end > 0) {
+    g.win_lo = end - 1 >= a.ori_win_left ? end - 1 - a.ori_win_left : 0;
+    g.n_win = end - g.win_lo;
+  }
+  if (a.scenario >= 2) {
+    g.thr = a.ratio.div(end);
+    g.n_cmp = a.scenario == 3 && a.topk < g.thr ? a.topk : g.thr;
+  }
+  return g;
+}
+
+// Positions [c0, c0 + clen) of an item's list -> cache rows in LDS (rowid: row number,
+// bit 31 set for the compressed cache, ROW_INVALID for masked positions; tmask: valid
+// bits of each 32-row tile), by a workgroup of NT threads; entries past the last tile
+// pair are left alone. Two dependent round trips at most (top-k ids, table words),
+// each with all its loads in flight; landed() runs when the words have arrived.
+//
+// Scenario 3 stops at the first -1 among the scanned top-k slots (golden.py:48-53).
+// The first chunk's own top-k loads double as the scan of its range; the slots
+// outside it are loaded in the same batch, and the table loads are issued before the
+// barrier that publishes the result (the cut is applied when the row ids are
+// packed). The two first_neg slots alternate between scans, so a slot is reset
+// without a barrier of its own.
+//
+// A short call spends most of its time up to its first row loads on instructions, not
+// on memory: a 32-bit division by a number in a register is some 30 of them, 64 bits
+// 100. Dividing by multiplication, leaving out positions past the list, forming row
+// numbers once and reading arguments per phase (fresh_args) took the way from the
+// kernel's entry to its first tile from 15.7 k to 13.2 k clocks (32 x 64-head window
+// decode; that kernel 14.8 -> 13.7 us, MLA decode with two rows 110.5 -> 107.6,
+// 13 sequences of fp8 rows with fp8 query products 41.5 -> 38.0, 8K prefill with
+// top-k 1086 -> 1060).
+struct Resolver {
+  ItemGeom g;
+  const int32_t *ori_tab, *cmp_tab;  // the batch's block-table rows (without a compressed
+  int cmp_len;                       // cache the raw one again, whose words are not used)
+  const int32_t* idx_row;            // the token's top-k ids, or null
+  bool tok_ok;
+  int jmax;                          // top-k slots to scan
+  bool stop_pending;
+  int cmp_stop;
+
+  __device__ Resolver(const KernelArgs& a, const ItemGeom& geom, int b, int tok, bool ok, int p_hi)
+      : g(geom), tok_ok(ok) {
+    ori_tab = a.ori_block_table + (size_t)b * a.ori_table_len;
+    cmp_tab = a.scenario >= 2 ? a.cmp_block_table + (size_t)b * a.cmp_table_len : ori_tab;
+    cmp_len = a.scenario >= 2 ? a.cmp_table_len : a.ori_table_len;
+    idx_row = a.scenario == 3 && a.cmp_indices && a.topk > 0
+                  ? a.cmp_indices + (size_t)(ok ? tok : 0) * a.topk : nullptr;
+    jmax = idx_row && p_hi > g.n_win ? min(p_hi - g.n_win, g.n_cmp) : 0;
+    stop_pending = jmax > 0;
+    cmp_stop = g.n_cmp;
+  }
+
+  template <int NT, int RCH, int LOADS, typename Landed>
+  __device__ __forceinline__ void chunk(const KernelArgs& a, int c0, int clen, int tid,
+                                        uint32_t* rowid, uint32_t* tmask, int* first_neg,
+                                        int& item_par, Landed&& landed) {
+    constexpr int PER = RCH / NT;              // positions per thread
+    constexpr int SCAN_PER = LOADS - PER;      // slots outside the chunk in the first batch
+    auto wanted = [&](int e) { return e == 0 || e * NT < clen + 2 * TILE; };  // uniform
+    int cid[PER], word[PER], off[PER], sv0[SCAN_PER];
+    const int own_lo = max(c0 - g.n_win, 0);
+    const int own_hi = min(max(c0 + clen - g.n_win, own_lo), jmax);
+    const int n_extra = stop_pending ? jmax - (own_hi - own_lo) : 0;
+    auto extra_slot = [&](int x) { return x < own_lo ? x : x + (own_hi - own_lo); };
+    if (idx_row) {
+      // all loads issued and waited for in one asm statement (gather_dwords_wait)
+      const int32_t* src[LOADS];
+      int got[LOADS];
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        const int jj = c0 + e * NT + tid - g.n_win;
+        src[e] = idx_row + (jj < 0 ? 0 : (jj < a.topk ? jj : a.topk - 1));
+      }
+#pragma unroll
+      for (int e = 0; e < SCAN_PER; ++e) {
+        const int x = e * NT + tid;  // clamped into range; unused when n_extra == 0
+        const int xc = x < n_extra ? x : (n_extra > 0 ? n_extra - 1 : 0);
+        src[PER + e] = idx_row + (n_extra > 0 ? extra_slot(xc) : 0);
+      }
+      gather_dwords_wait(got, src);
+#pragma unroll
+      for (int e = 0; e < SCAN_PER; ++e) sv0[e] = got[PER + e];
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        const int r = e * NT + tid;
+        cid[e] = (r < clen && tok_ok && c0 + r >= g.n_win) ? got[e] : -1;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < PER; ++e) cid[e] = tok_ok ? c0 + e * NT + tid - g.n_win : -1;
+    }
+    if (stop_pending) {
+      int mine = g.n_cmp;
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        const int jj = c0 + e * NT + tid - g.n_win;
+        if (jj >= 0 && jj < jmax && e * NT + tid < clen && cid[e] == -1 && jj < mine) mine = jj;
+      }
+#pragma unroll
+      for (int e = 0; e < SCAN_PER; ++e) {
+        const int x = e * NT + tid;
+        if (x < n_extra && sv0[e] == -1 && extra_slot(x) < mine) mine = extra_slot(x);
+      }
+      for (int x0 = NT * SCAN_PER; x0 < n_extra; x0 += NT * SCAN_PER) {  // beyond the first round
+        int v[SCAN_PER];
+#pragma unroll
+        for (int e = 0; e < SCAN_PER; ++e) {  // unconditional, clamped: all loads in flight at once
+          const int x = x0 + e * NT + tid;
+          v[e] = idx_row[extra_slot(x < n_extra ? x : n_extra - 1)];
+        }
+#pragma unroll
+        for (int e = 0; e < SCAN_PER; ++e) {
+          const int x = x0 + e * NT + tid;
+          if (x < n_extra && v[e] == -1 && extra_slot(x) < mine) mine = extra_slot(x);
+        }
+      }
+      if (mine < g.n_cmp) atomicMin(&first_neg[item_par], mine);
+    }
+    // block-table words (compiler-visible loads with in-bounds addresses); off: the
+    // position's row within its block, -1 when it has none
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      word[e] = off[e] = -1;
+      if (!wanted(e)) continue;
+      const int r = e * NT + tid;
+      const bool win = c0 + r < g.n_win;
+      const int key = win ? g.win_lo + c0 + r : cid[e];
+      const int tlen = win ? a.ori_table_len : cmp_len;  // >= 1
+      const FastDiv bs = {win ? a.ori_bs.mul : a.cmp_bs.mul, win ? a.ori_bs.shift : a.cmp_bs.shift};
+      const int bi = key >= 0 ? bs.div(key) : 0;
+      word[e] = (win ? ori_tab : cmp_tab)[bi < tlen ? bi : tlen - 1];
+      if (r < clen && tok_ok && key >= 0 && bi < tlen && (win || key < g.thr))
+        off[e] = key - bi * (win ? a.ori_block_size : a.cmp_block_size);
+    }
+    // every load so far (table words, query fragment) has landed, as the compiler sees it
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0) expcnt(7) lgkmcnt(15)
+    landed();
+    if (stop_pending) {
+      __syncthreads();  // every thread's atomicMin is in
+      cmp_stop = min(first_neg[item_par], g.n_cmp);
+      if (tid == 0) first_neg[item_par ^ 1] = INT32_MAX;  // the next scan's slot
+      item_par ^= 1;
+      stop_pending = false;
+    }
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      if (!wanted(e)) continue;
+      const int r = e * NT + tid;
+      const bool win = c0 + r < g.n_win;
+      const bool ok = off[e] >= 0 && word[e] >= 0 &&
+                      word[e] < (win ? a.ori_block_num : a.cmp_block_num) &&
+                      (win || c0 + r - g.n_win < cmp_stop);
+      const int row = word[e] * (win ? a.ori_block_size : a.cmp_block_size) + off[e];
+      // masked rows are read from the zero row
+      rowid[r] = ok ? (uint32_t)row | (win ? 0u : 0x80000000u) : ROW_INVALID;
+      const unsigned long long bal = __ballot(ok);
+      if ((tid & 63) == 0) {
+        tmask[r / TILE] = (uint32_t)bal;
+        tmask[r / TILE + 1] = (uint32_t)(bal >> 32);
+      }
+    }
+    __syncthreads();
+  }
+};
+
+// Rows [0, nh) of a staging area of ROWS rows (SROW bytes apart, 1 KB each) to global
+// memory, one row per store instruction: wave w of NW takes rows w, w + NW, ..., a
+// batch read from LDS before it is stored. put(h, v): lane's 16 bytes of row h.
+template <int ROWS, int NW, int SROW, typename Put>
+__device__ __forceinline__ void rows_out(const unsigned char* stg, int nh, int w, int lane,
+                                         Put&& put) {
+  constexpr int N = ROWS / NW, BATCH = N < 8 ? N : 8;
+  static_assert(ROWS % NW == 0 && N % BATCH == 0, "rows per wave");
+#pragma unroll
+  for (int k0 = 0; k0 < N; k0 += BATCH) {
+    i32x4 v[BATCH];
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k)
+      v[k] = *(const i32x4*)(stg + (w + NW * (k0 + k)) * SROW + 16 * lane);
+#pragma unroll
+    for (int k = 0; k < BATCH; ++k)
+      if (w + NW * (k0 + k) < nh) put(w + NW * (k0 + k), v[k]);
+  }
+}
+
 // Device-built schedules (num_fd == SAS_SCHED_DEVICE): the summary is read from
 // the metadata config row; num_fa and num_partial_slots are the launch and
 // workspace capacities it must fit.
@@ -405,8 +636,10 @@ __device__ void merge_item_here(const SasAttnArgs& a, int tok, int hb, int slot0
   constexpr int G = HPW < 8 ? HPW : 8;  // heads per group
   constexpr int PB = 2;                 // pieces per batch of loads
   static_assert(DV == 512 && MB % NW == 0 && HPW % G == 0 && HPW <= 64, "merge layout");
-  const int lane = threadIdx.x & 63;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // (nothing of the merge is formed before its call)
+  const int lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nh = min(MB, a.num_heads - hb * MB);
   const int hw0 = w * HPW;
   if (hw0 >= nh) return;
@@ -591,7 +824,7 @@ __device__ inline void quantize_q(const i16x8 (&qf)[18], i32x8 (&q8)[4], float& 
 // fragment during the current item's epilogue. Decode launches keep the
 // simpler first-chunk load (measured faster for their short items).
 template <int DQK, int DV, int NHG, typename T, int KVF, bool PREF>
-__global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
+__global__ __launch_bounds__(128 * NHG) void attn2_kernel(const KernelArgs a) {
   constexpr int NW = 2 * NHG;            // waves per workgroup
   constexpr int MB = 32 * NHG;           // heads per item (m-block)
   constexpr int NT = 64 * NW;            // threads
@@ -629,7 +862,8 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
   const int dh = w / NHG;
   const int partner = w ^ NHG;
   const int hlocal = hg * 32 + (lane & 31);  // head within the item's m-block
-  const int hblocks = (a.num_heads + MB - 1) / MB;
+  const int hblocks = (a.num_heads + MB - 1) / MB;  // 1 or 2 (the launch's check of m_base)
+  const int hshift = hblocks - 1;
   const int hl = lane >> 5;
   // Kᵀ operand: row lane%32, main chunk 32dh + 2ks + hl (dims 256dh + 16ks + 8hl),
   // rope chunk 4dh + 2(ks - 16) + hl
@@ -643,6 +877,18 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
   const int tr_base = main_row_base(4 * hl + ((lane & 15) >> 2)) + dh * DV +
                       ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
 
+  // With at most 64 batches, every batch's lengths and query offset sit in one
+  // lane each, loaded at the start beside the metadata row (they no longer wait
+  // for it: the item's batch picks its lane).
+  const QRows qrows(a);
+  const bool lens_in_lanes = a.batch <= 64;
+  int lane_aq = 0, lane_kv = 0, lane_qp = 0;
+  if (lens_in_lanes) {
+    const int lb = lane < a.batch ? lane : a.batch - 1;
+    lane_aq = qrows.rows[lb];
+    lane_kv = a.seqused_kv[lb];
+    lane_qp = qrows.first[lb];
+  }
   int s2b = a.s2_base;
   int nfa = a.num_fa;
   if (a.num_fd == SAS_SCHED_DEVICE) {
@@ -661,7 +907,7 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
   if (fa[0] == 0) return;
   // where the whole schedule ends (loaded beside this row's cursors)
   const int32_t* fa_last = a.metadata + (nfa - 1) * SAS_FA_METADATA_SIZE;
-  const int last_b = fa_last[4] < a.batch ? fa_last[4] : a.batch;
+  const int last_b = fa_last[4] < 0 ? 0 : (fa_last[4] < a.batch ? fa_last[4] : a.batch);
   const int last_m = fa_last[4] < a.batch ? fa_last[5] : 0;
   int b = fa[1], m = fa[2];
   const int j_start = fa[3];
@@ -677,18 +923,6 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
   const char* ori_kv = (const char*)a.ori_kv;
   const char* cmp_kv = (const char*)(a.cmp_kv ? a.cmp_kv : a.ori_kv);
   const float sc = a.softmax_scale * LOG2E;
-  // With at most 64 batches, every batch's lengths and query offset sit in one
-  // lane each, loaded at the start beside the metadata row (they no longer wait
-  // for it: the item's batch picks its lane).
-  const QRows qrows(a);
-  const bool lens_in_lanes = a.batch <= 64;
-  int lane_aq = 0, lane_kv = 0, lane_qp = 0;
-  if (lens_in_lanes) {
-    const int lb = lane < a.batch ? lane : a.batch - 1;
-    lane_aq = qrows.rows[lb];
-    lane_kv = a.seqused_kv[lb];
-    lane_qp = qrows.first[lb];
-  }
   if (tid < 2) first_neg[tid] = INT32_MAX;
   // piece index of the first item when it continues a split item
   const int cont_k = (merge_here && j_start > 0) ? continued_piece_index(a, fa_row, b, m, cscan) : 0;
@@ -711,7 +945,7 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
   int tok_lo = 0, tok_hi = a.total_tokens;
   if (qrows.cumulative) {
     tok_lo = ld_uniform(qrows.first);
-    tok_hi = ld_uniform(qrows.first + last_b) + last_m / ((a.num_heads + MB - 1) / MB);
+    tok_hi = ld_uniform(qrows.first + last_b) + (last_m >> hshift);
   }
   int item_par = 0;  // which first_neg slot the next top-k scan uses
   bool first_item = true;
@@ -734,7 +968,9 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
       qp = qrows.start(bc, first_b);
     }
   };
-  // this wave's query fragment of (token, head), zero for rows out of range
+  // this wave's query fragment of (token, head); rows out of range read token 0's
+  // first head: their scores only reach their own softmax column, never stored (and
+  // nothing here waits for the loads)
   auto load_q = [&](int qtok, int qhead) {
     const bool ok = qtok >= 0 && qtok < a.total_tokens && qhead < a.num_heads;
     const short* qrow = (const short*)a.q + ((size_t)(ok ? qtok : 0) * a.num_heads +
@@ -743,11 +979,11 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
     for (int ks = 0; ks < NKS; ++ks) {
       const int dim = ks < NKS_MAIN ? (256 * dh + 16 * ks + 8 * hl)
                                     : (512 + 32 * dh + 16 * (ks - NKS_MAIN) + 8 * hl);
-      i16x8 v = *(const i16x8*)(qrow + dim);
-      qf[ks] = ok ? v : (i16x8){0, 0, 0, 0, 0, 0, 0, 0};
+      qf[ks] = *(const i16x8*)(qrow + dim);
     }
   };
   for (;;) {
+    const KernelArgs a = fresh_args();
     const bool have_q = PREF && q_pref;
     q_pref = false;
     b = __builtin_amdgcn_readfirstlane(b);
@@ -762,22 +998,18 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
     }
     if (b >= a.batch || b > b_end || (b == b_end && m > s_end)) break;
     const bool is_end = (b == b_end && m == s_end);
-    const int s = m / hblocks;
+    const int s = m >> hshift;
     const int head = (m - s * hblocks) * MB + hlocal;
     const bool head_ok = head < a.num_heads;
     if (is_end && j_end == 0) break;
 
     const int tok = qpre + s;
-    const ItemGeom g =
-        item_geom(act_q, act_kv, s, a.ori_win_left, a.scenario, a.cmp_ratio, a.topk);
+    const ItemGeom g = item_geom_at(a, act_q, act_kv, s);
     const int L = g.n_win + g.n_cmp;
-    const int nblk = (L + s2b - 1) / s2b;
-    const int blo = first_item ? j_start : 0;
-    int bhi = is_end ? j_end : nblk;
-    if (bhi > nblk) bhi = nblk;
     const bool partial = (first_item && j_start > 0) || is_end;
+    const int blo = first_item ? j_start : 0;
     const int p_lo = blo * s2b;
-    const int p_hi = bhi * s2b < L ? bhi * s2b : L;
+    const int p_hi = is_end && (int64_t)j_end * s2b < L ? j_end * s2b : L;
     const bool tok_ok = tok >= 0 && tok < a.total_tokens;
 
     // ---- online-softmax state (golden.py:156-160 seeds m = sink, l = 1; the 1
@@ -802,7 +1034,7 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
       // other batches the early loads delayed this item's output stores by more
       // than they saved (SWA decode +4 %, A/B)
       if (nb != b) return false;
-      const int ns = nm / hblocks;
+      const int ns = nm >> hshift;
       load_q(qp + ns, (nm - ns * hblocks) * MB + hlocal);
       return true;
     };
@@ -819,20 +1051,7 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
 #pragma unroll
       for (int j = 0; j < 16; ++j) acc[d][j] = 0.0f;
 
-    // ---- scenario 3: position of the first -1 among the scanned top-k slots ----
-    // (golden.py:48-53: the scan stops at the first -1). The first chunk's own
-    // top-k loads double as the scan of its range; the slots outside it are
-    // loaded in the same batch, and the block-table loads of the chunk are
-    // issued before the barrier that publishes the result (the -1 cut is
-    // applied when the row ids are packed). The two first_neg slots alternate
-    // between scans, so a slot is reset without a barrier of its own.
-    const int32_t* idx_row =
-        a.cmp_indices ? a.cmp_indices + (size_t)(tok_ok ? tok : 0) * a.topk : nullptr;
-    const bool scan3 = a.scenario == 3 && idx_row != nullptr && a.topk > 0;
-    const int jmax = (scan3 && p_hi > g.n_win) ? min(p_hi - g.n_win, g.n_cmp) : 0;
-    bool stop_pending = jmax > 0;
-    int cmp_stop = g.n_cmp;
-
+    Resolver res(a, g, b, tok, tok_ok, p_hi);
     for (int c0 = p_lo; c0 < p_hi; c0 += RCH) {
       const int clen = (p_hi - c0) < RCH ? (p_hi - c0) : RCH;
       const int ntile = (clen + TILE - 1) / TILE;
@@ -841,126 +1060,10 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
       // loads, so they land during its memory round trips; the compiler's wait
       // for the table words below covers them
       if (c0 == p_lo && !have_q) load_q(tok, head);
-      // ---- resolve positions -> cache rows (bit 31: compressed cache) ----
-      constexpr int PER = RCH / NT;
-      static_assert(PER == 4, "resolution positions per thread");
-      int cid[PER];
-      int tab[PER];
-      const int own_lo = max(c0 - g.n_win, 0);
-      const int own_hi = min(max(c0 + clen - g.n_win, own_lo), jmax);
-      const int n_extra = stop_pending ? jmax - (own_hi - own_lo) : 0;
-      constexpr int SCAN_PER = 4;
-      auto extra_slot = [&](int x) { return x < own_lo ? x : x + (own_hi - own_lo); };
-      int sv0[SCAN_PER];
-      if (scan3) {
-        // all loads issued and waited for in one asm statement (gather_dwords_wait)
-        int v[PER];
-        const int32_t* src[PER + SCAN_PER];
-        int got[PER + SCAN_PER];
-#pragma unroll
-        for (int e = 0; e < PER; ++e) {
-          const int jj = c0 + e * NT + tid - g.n_win;
-          src[e] = idx_row + (jj < 0 ? 0 : (jj < a.topk ? jj : a.topk - 1));
-        }
-#pragma unroll
-        for (int e = 0; e < SCAN_PER; ++e) {
-          const int x = e * NT + tid;  // clamped into range; unused when n_extra == 0
-          const int xc = x < n_extra ? x : (n_extra > 0 ? n_extra - 1 : 0);
-          src[PER + e] = idx_row + (n_extra > 0 ? extra_slot(xc) : 0);
-        }
-        gather_dwords_wait(got, src);
-#pragma unroll
-        for (int e = 0; e < PER; ++e) v[e] = got[e];
-#pragma unroll
-        for (int e = 0; e < SCAN_PER; ++e) sv0[e] = got[PER + e];
-#pragma unroll
-        for (int e = 0; e < PER; ++e) {
-          const int r = e * NT + tid;
-          const int pos = c0 + r;
-          cid[e] = (r < clen && tok_ok && pos >= g.n_win) ? v[e] : -1;
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < PER; ++e) {
-          const int r = e * NT + tid;
-          const int pos = c0 + r;
-          cid[e] = (r < clen && tok_ok && pos >= g.n_win) ? pos - g.n_win : -1;
-        }
-      }
-      if (stop_pending) {
-        int mine = g.n_cmp;
-#pragma unroll
-        for (int e = 0; e < PER; ++e) {
-          const int jj = c0 + e * NT + tid - g.n_win;
-          if (jj >= 0 && jj < jmax && e * NT + tid < clen && cid[e] == -1 && jj < mine) mine = jj;
-        }
-#pragma unroll
-        for (int e = 0; e < SCAN_PER; ++e) {
-          const int x = e * NT + tid;
-          if (x < n_extra && sv0[e] == -1 && extra_slot(x) < mine) mine = extra_slot(x);
-        }
-        for (int x0 = NT * SCAN_PER; x0 < n_extra; x0 += NT * SCAN_PER) {  // beyond the first round
-          int v[SCAN_PER];
-#pragma unroll
-          for (int e = 0; e < SCAN_PER; ++e) {  // unconditional, clamped: all loads in flight at once
-            const int x = x0 + e * NT + tid;
-            v[e] = idx_row[extra_slot(x < n_extra ? x : n_extra - 1)];
-          }
-#pragma unroll
-          for (int e = 0; e < SCAN_PER; ++e) {
-            const int x = x0 + e * NT + tid;
-            if (x < n_extra && v[e] == -1 && extra_slot(x) < mine) mine = extra_slot(x);
-          }
-        }
-        if (mine < g.n_cmp) atomicMin(&first_neg[item_par], mine);
-      }
-      // block-table words (compiler-visible loads with in-bounds addresses)
-#pragma unroll
-      for (int e = 0; e < PER; ++e) {
-        const int r = e * NT + tid;
-        const int pos = c0 + r;
-        const bool win = pos < g.n_win;
-        const int key = win ? g.win_lo + pos : cid[e];
-        const int bsz = win ? a.ori_block_size : a.cmp_block_size;
-        const int tlen = win ? a.ori_table_len : a.cmp_table_len;
-        const int32_t* tbl = win ? a.ori_block_table : a.cmp_block_table;
-        const int bi = key >= 0 ? key / bsz : 0;
-        const bool ok = r < clen && tok_ok && key >= 0 && bi < tlen && (win || cid[e] < g.thr);
-        const int t = (tbl != nullptr) ? tbl[(size_t)b * tlen + (bi < tlen ? bi : tlen - 1)] : -1;
-        tab[e] = ok ? t : -1;
-      }
-      // every load so far (table words, query fragment) has landed, as the compiler sees it
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0) expcnt(7) lgkmcnt(15)
-      if (c0 == p_lo) m_run = seed_m();
-      if (stop_pending) {
-        __syncthreads();  // every thread's atomicMin is in
-        cmp_stop = min(first_neg[item_par], g.n_cmp);
-        if (tid == 0) first_neg[item_par ^ 1] = INT32_MAX;  // the next scan's slot
-        item_par ^= 1;
-        stop_pending = false;
-      }
-#pragma unroll
-      for (int e = 0; e < PER; ++e) {
-        const int r = e * NT + tid;
-        const int pos = c0 + r;
-        uint32_t id = ROW_INVALID;
-        const int phys = tab[e];
-        if (r < clen && tok_ok && phys >= 0) {
-          if (pos < g.n_win) {
-            if (phys < a.ori_block_num)
-              id = (uint32_t)(phys * a.ori_block_size + (g.win_lo + pos) % a.ori_block_size);
-          } else if (phys < a.cmp_block_num && (!scan3 || pos - g.n_win < cmp_stop)) {
-            id = (uint32_t)(phys * a.cmp_block_size + cid[e] % a.cmp_block_size) | 0x80000000u;
-          }
-        }
-        rowid[r] = id;  // masked rows are read from the zero row
-        const unsigned long long bal = __ballot(id != ROW_INVALID);
-        if (lane == 0) {
-          tmask[(r - lane) / TILE] = (uint32_t)bal;
-          tmask[(r - lane) / TILE + 1] = (uint32_t)(bal >> 32);
-        }
-      }
-      __syncthreads();
+      // ---- positions -> cache rows (bit 31: compressed cache) ----
+      res.template chunk<NT, RCH, 8>(a, c0, clen, tid, rowid, tmask, first_neg, item_par, [&] {
+        if (c0 == p_lo) m_run = seed_m();
+      });
 
       // ---- DMA issue for one tile into one ring stage ----
       // main part: wave w fills rows w, w + NW, ...; one 1 KB row per instruction
@@ -1271,13 +1374,15 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
     // whole rows ----
     __syncthreads();
     {
+      const KernelArgs a = fresh_args();
+      int w_e = w;  // (the rows' addresses are formed here, not before the item loop)
+      asm volatile("" : "+s"(w_e));
       unsigned char* stg = kv_lds;
       const int nh = min(MB, a.num_heads - hb * MB);  // heads of this item
-      int tid_e = tid, hl_e = hlocal, dv_e = dh * (DV / 2) + 4 * hl;
-      asm volatile("" : "+v"(tid_e), "+v"(hl_e), "+v"(dv_e));
+      int lane_e = lane, hl_e = hlocal, dv_e = dh * (DV / 2) + 4 * hl;
+      asm volatile("" : "+v"(lane_e), "+v"(hl_e), "+v"(dv_e));
       if (!partial) {
         constexpr int SROW = DV * 2 + 16;  // staging row stride (bytes; 16-byte aligned rows)
-        constexpr int CPR = DV * 2 / 16;   // 16-byte chunks per row
         static_assert(MB * SROW <= NSTG * STAGE_BYTES, "output staging");
         const float inv = 1.0f / l_run;
 #pragma unroll
@@ -1294,10 +1399,9 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
         __syncthreads();
         if (tok_ok) {
           char* obase = (char*)((T*)a.out + ((size_t)tok * a.num_heads + hb * MB) * DV);
-          for (int c = tid_e; c < nh * CPR; c += NT) {
-            const int h = c / CPR, c16 = c - h * CPR;
-            *(i16x8*)(obase + (size_t)h * DV * 2 + c16 * 16) = *(const i16x8*)(stg + h * SROW + c16 * 16);
-          }
+          rows_out<MB, NW, SROW>(stg, nh, w_e, lane_e, [&](int h, i32x4 v) {
+            *(i32x4*)(obase + h * DV * 2 + 16 * lane_e) = v;
+          });
           if (dh == 0 && hl == 0 && head_ok)
             a.lse[(size_t)tok * a.num_heads + hb * MB + hl_e] = (m_run + __log2f(l_run)) * LN2;
         }
@@ -1306,7 +1410,6 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
         // l, l ^ 32 and the partner wave) picks the scale; rows staged whole, as
         // the outputs are
         constexpr int SROW = DV * 2 + 16;  // staging row stride (bytes; 16-byte aligned rows)
-        constexpr int CPR = DV * 2 / 16;   // 16-byte chunks per row
         static_assert(MB * SROW + 2 * MB * 4 <= NSTG * STAGE_BYTES, "partial staging");
         float* rmax = (float*)(stg + MB * SROW);
         const bool empty = !(l_run > 0.0f);
@@ -1338,11 +1441,9 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
           // read by another workgroup in this launch: agent-coherent stores
           const __amdgpu_buffer_rsrc_t rs = partial_rsrc(a, MB, DV);
           const uint32_t base = (uint32_t)slot * MB * DV * 2;
-          for (int c = tid_e; c < nh * CPR; c += NT) {
-            const int h = c / CPR, c16 = c - h * CPR;
-            partial_store16(rs, base + (uint32_t)(h * DV * 2 + c16 * 16),
-                            *(const i32x4*)(stg + h * SROW + c16 * 16));
-          }
+          rows_out<MB, NW, SROW>(stg, nh, w_e, lane_e, [&](int h, i32x4 v) {
+            partial_store16(rs, base + (uint32_t)(h * DV * 2 + 16 * lane_e), v);
+          });
           if (dh == 0 && hl == 0 && head_ok) {
             const uint32_t lo = (uint32_t)a.num_partial_slots * MB * DV * 2;
             partial_store4(rs, lo + ((uint32_t)slot * MB + hl_e) * 4, lse_piece);
@@ -1351,11 +1452,9 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
           }
         } else {
           char* wbase = (char*)a.workspace + (size_t)slot * MB * DV * 2;
-          for (int c = tid_e; c < nh * CPR; c += NT) {
-            const int h = c / CPR, c16 = c - h * CPR;
-            *(i16x8*)(wbase + (size_t)h * DV * 2 + c16 * 16) =
-                *(const i16x8*)(stg + h * SROW + c16 * 16);
-          }
+          rows_out<MB, NW, SROW>(stg, nh, w_e, lane_e, [&](int h, i32x4 v) {
+            *(i32x4*)(wbase + h * DV * 2 + 16 * lane_e) = v;
+          });
           if (dh == 0 && hl == 0 && head_ok) {
             float* wl = partial_lse(a, MB, DV);
             wl[(size_t)slot * MB + hl_e] = lse_piece;
@@ -1366,8 +1465,10 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const SasAttnArgs a) {
     }
     if (partial && merge_here) {
       // the piece that completes the item merges it (bit-identical to merge_kernel)
+      const KernelArgs a = fresh_args();
       const int slot0 = (first_item && j_start > 0) ? slot - cont_k : slot;
       if (slot0 >= 0 && slot < a.num_partial_slots && slot0 < SAS_MERGE_SYNC_WORDS) {
+        const int nblk = (L + s2b - 1) / s2b, bhi = p_hi < L ? j_end : nblk;
         const int npc = split_arrive(a, slot0, slot, bhi - blo, bhi == nblk, nblk, &merge_word);
         if (npc > 0) merge_item_here<DV, T, MB, NW>(a, tok, hb, slot0, npc);
       }
@@ -1438,7 +1539,7 @@ __device__ __host__ inline int k8_swz(int r) {
 __device__ __host__ inline int k8_chunk(int r, int c) { return (c & 16) | ((c ^ k8_swz(r)) & 15); }
 
 template <int DQK, int DV, int NHG, typename T, int KVF, bool QK8 = false>
-__global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
+__global__ __launch_bounds__(256 * NHG) void attn3_kernel(const KernelArgs a) {
   constexpr int NW = 4 * NHG;            // waves per workgroup
   constexpr int MB = 32 * NHG;           // heads per item (m-block)
   constexpr int NT = 64 * NW;            // threads
@@ -1503,7 +1604,8 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
   const int hq = hg * 32 + 16 * qh + r16;    // softmax head within the m-block
   const int hp = hg * 32 + (lane & 31);      // P·V head within the m-block
   const bool has_rope = ROPE && w < NROPE;   // this wave issues rope DMA instruction w
-  const int hblocks = (a.num_heads + MB - 1) / MB;
+  const int hblocks = (a.num_heads + MB - 1) / MB;  // 1 or 2 (the launch's check of m_base)
+  const int hshift = hblocks - 1;
   // Kᵀ operand of 16x16x32 (A = 16 rows x 32 dims): row 16rh + r16, dims 32ks + 8g4
   const int k_row = 16 * rh + r16;
   const int k_base = ring_row_base(k_row) + 16 * g4;
@@ -1532,6 +1634,16 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
   const int pr_off0 = hg * PB_HG + pr_head * 64 + 16 * ((0 + hl) ^ ((pr_head >> 2) & 3));
   const int pr_off1 = hg * PB_HG + pr_head * 64 + 16 * ((2 + hl) ^ ((pr_head >> 2) & 3));
 
+  // with at most 64 batches, their lengths and query offsets in one lane each
+  const QRows qrows(a);
+  const bool lens_in_lanes = a.batch <= 64;
+  int lane_aq = 0, lane_kv = 0, lane_qp = 0;
+  if (lens_in_lanes) {
+    const int lb = lane < a.batch ? lane : a.batch - 1;
+    lane_aq = qrows.rows[lb];
+    lane_kv = a.seqused_kv[lb];
+    lane_qp = qrows.first[lb];
+  }
   int s2b = a.s2_base;
   int nfa = a.num_fa;
   if (a.num_fd == SAS_SCHED_DEVICE) {
@@ -1550,7 +1662,7 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
   if (fa[0] == 0) return;
   // where the whole schedule ends (loaded beside this row's cursors)
   const int32_t* fa_last = a.metadata + (nfa - 1) * SAS_FA_METADATA_SIZE;
-  const int last_b = fa_last[4] < a.batch ? fa_last[4] : a.batch;
+  const int last_b = fa_last[4] < 0 ? 0 : (fa_last[4] < a.batch ? fa_last[4] : a.batch);
   const int last_m = fa_last[4] < a.batch ? fa_last[5] : 0;
   int b = fa[1], m = fa[2];
   const int j_start = fa[3];
@@ -1564,12 +1676,14 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
   if (tid < 2) first_neg[tid] = INT32_MAX;
   __syncthreads();
 
-  const QRows qrows(a);
+  lane_aq = qrows.count(lane_aq, lane_qp);
+  lane_qp = qrows.start(lane, lane_qp);
+  asm volatile("" : "+v"(lane_aq), "+v"(lane_kv), "+v"(lane_qp));
   // cumulative row counts: the tokens [tok_lo, tok_hi) of the schedule's rows
   int tok_lo = 0, tok_hi = a.total_tokens;
   if (qrows.cumulative) {
     tok_lo = ld_uniform(qrows.first);
-    tok_hi = ld_uniform(qrows.first + last_b) + last_m / ((a.num_heads + MB - 1) / MB);
+    tok_hi = ld_uniform(qrows.first + last_b) + (last_m >> hshift);
   }
 
   // Sinks of this lane's softmax head in the (at most two) head blocks of an
@@ -1581,6 +1695,7 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
   int item_par = 0;  // which first_neg slot the next top-k scan uses
   bool first_item = true;
   for (;;) {
+    const KernelArgs a = fresh_args();
     b = __builtin_amdgcn_readfirstlane(b);
     m = __builtin_amdgcn_readfirstlane(m);
     // the batch's lengths and query offset, loaded together (one scalar round
@@ -1588,6 +1703,12 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
     int act_q, act_kv, qpre;
     auto load_batch = [&] {
       const int bc = b < a.batch ? b : a.batch - 1;
+      if (lens_in_lanes) {
+        act_q = __builtin_amdgcn_readlane(lane_aq, bc);
+        act_kv = __builtin_amdgcn_readlane(lane_kv, bc);
+        qpre = __builtin_amdgcn_readlane(lane_qp, bc);
+        return;
+      }
       const int first_b = ld_uniform(qrows.first + bc);
       act_q = qrows.count(ld_uniform(qrows.rows + bc), first_b);
       act_kv = ld_uniform(a.seqused_kv + bc);
@@ -1602,21 +1723,17 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
     }
     if (b >= a.batch || b > b_end || (b == b_end && m > s_end)) break;
     const bool is_end = (b == b_end && m == s_end);
-    const int s = m / hblocks;
+    const int s = m >> hshift;
     const int hb = m - s * hblocks;
     if (is_end && j_end == 0) break;
 
     const int tok = qpre + s;
-    const ItemGeom g =
-        item_geom(act_q, act_kv, s, a.ori_win_left, a.scenario, a.cmp_ratio, a.topk);
+    const ItemGeom g = item_geom_at(a, act_q, act_kv, s);
     const int L = g.n_win + g.n_cmp;
-    const int nblk = (L + s2b - 1) / s2b;
-    const int blo = first_item ? j_start : 0;
-    int bhi = is_end ? j_end : nblk;
-    if (bhi > nblk) bhi = nblk;
     const bool partial = (first_item && j_start > 0) || is_end;
+    const int blo = first_item ? j_start : 0;
     const int p_lo = blo * s2b;
-    const int p_hi = bhi * s2b < L ? bhi * s2b : L;
+    const int p_hi = is_end && (int64_t)j_end * s2b < L ? j_end * s2b : L;
     const bool tok_ok = tok >= 0 && tok < a.total_tokens;
 
     // query fragment of the wave's 16 heads (B operand of Sᵀ = K·Qᵀ)
@@ -1643,20 +1760,7 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
 #pragma unroll
       for (int j = 0; j < 16; ++j) acc[d][j] = 0.0f;
 
-    // ---- scenario 3: position of the first -1 among the scanned top-k slots ----
-    // (golden.py:48-53: the scan stops at the first -1). The first chunk's own
-    // top-k loads double as the scan of its range; the slots outside it are
-    // loaded in the same batch, and the block-table loads of the chunk are
-    // issued before the barrier that publishes the result (the -1 cut is
-    // applied when the row ids are packed). The two first_neg slots alternate
-    // between scans, so a slot is reset without a barrier of its own.
-    const int32_t* idx_row =
-        a.cmp_indices ? a.cmp_indices + (size_t)(tok_ok ? tok : 0) * a.topk : nullptr;
-    const bool scan3 = a.scenario == 3 && idx_row != nullptr && a.topk > 0;
-    const int jmax = (scan3 && p_hi > g.n_win) ? min(p_hi - g.n_win, g.n_cmp) : 0;
-    bool stop_pending = jmax > 0;
-    int cmp_stop = g.n_cmp;
-
+    Resolver res(a, g, b, tok, tok_ok, p_hi);
     for (int c0 = p_lo; c0 < p_hi; c0 += RCH) {
       const int clen = (p_hi - c0) < RCH ? (p_hi - c0) : RCH;
       const int ntile = (clen + TILE - 1) / TILE;
@@ -1669,7 +1773,8 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
       if (QK8 || c0 == p_lo) {
         const int head_q = hb * MB + hq;
         const bool hok = head_q < a.num_heads && tok_ok;
-        const short* qrow = (const short*)a.q + ((size_t)(tok_ok ? tok : 0) * a.num_heads +
+        // (rows out of range read token 0's first head: never stored)
+        const short* qrow = (const short*)a.q + ((size_t)(hok ? tok : 0) * a.num_heads +
                                                  (hok ? head_q : 0)) * DQK;
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) {
@@ -1677,133 +1782,14 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
           // lane's quarter of e4m3 block blk)
           const int dim = (QK8 && ks < NKS_MAIN) ? 128 * (ks >> 2) + 32 * g4 + 8 * (ks & 3)
                                                  : 32 * ks + 8 * g4;
-          i16x8 v = *(const i16x8*)(qrow + dim);
-          qf[ks] = hok ? v : (i16x8){0, 0, 0, 0, 0, 0, 0, 0};
+          qf[ks] = *(const i16x8*)(qrow + dim);
         }
       }
-      // ---- resolve positions -> cache rows (bit 31: compressed cache) ----
-      constexpr int PER = RCH / NT;
-      static_assert(PER == 2 || PER == 4, "resolution positions per thread");
-      int cid[PER];
-      int tab[PER];
-      const int own_lo = max(c0 - g.n_win, 0);
-      const int own_hi = min(max(c0 + clen - g.n_win, own_lo), jmax);
-      const int n_extra = stop_pending ? jmax - (own_hi - own_lo) : 0;
-      constexpr int SCAN_PER = 4;
-      auto extra_slot = [&](int x) { return x < own_lo ? x : x + (own_hi - own_lo); };
-      int sv0[SCAN_PER];
-      if (scan3) {
-        // all loads issued and waited for in one asm statement (gather_dwords_wait)
-        int v[PER];
-        const int32_t* src[PER + SCAN_PER];
-        int got[PER + SCAN_PER];
-#pragma unroll
-        for (int e = 0; e < PER; ++e) {
-          const int jj = c0 + e * NT + tid - g.n_win;
-          src[e] = idx_row + (jj < 0 ? 0 : (jj < a.topk ? jj : a.topk - 1));
-        }
-#pragma unroll
-        for (int e = 0; e < SCAN_PER; ++e) {
-          const int x = e * NT + tid;  // clamped into range; unused when n_extra == 0
-          const int xc = x < n_extra ? x : (n_extra > 0 ? n_extra - 1 : 0);
-          src[PER + e] = idx_row + (n_extra > 0 ? extra_slot(xc) : 0);
-        }
-        gather_dwords_wait(got, src);
-#pragma unroll
-        for (int e = 0; e < PER; ++e) v[e] = got[e];
-#pragma unroll
-        for (int e = 0; e < SCAN_PER; ++e) sv0[e] = got[PER + e];
-#pragma unroll
-        for (int e = 0; e < PER; ++e) {
-          const int r = e * NT + tid;
-          const int pos = c0 + r;
-          cid[e] = (r < clen && tok_ok && pos >= g.n_win) ? v[e] : -1;
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < PER; ++e) {
-          const int r = e * NT + tid;
-          const int pos = c0 + r;
-          cid[e] = (r < clen && tok_ok && pos >= g.n_win) ? pos - g.n_win : -1;
-        }
-      }
-      if (stop_pending) {
-        int mine = g.n_cmp;
-#pragma unroll
-        for (int e = 0; e < PER; ++e) {
-          const int jj = c0 + e * NT + tid - g.n_win;
-          if (jj >= 0 && jj < jmax && e * NT + tid < clen && cid[e] == -1 && jj < mine) mine = jj;
-        }
-#pragma unroll
-        for (int e = 0; e < SCAN_PER; ++e) {
-          const int x = e * NT + tid;
-          if (x < n_extra && sv0[e] == -1 && extra_slot(x) < mine) mine = extra_slot(x);
-        }
-        for (int x0 = NT * SCAN_PER; x0 < n_extra; x0 += NT * SCAN_PER) {  // beyond the first round
-          int v[SCAN_PER];
-#pragma unroll
-          for (int e = 0; e < SCAN_PER; ++e) {  // unconditional, clamped: all loads in flight at once
-            const int x = x0 + e * NT + tid;
-            v[e] = idx_row[extra_slot(x < n_extra ? x : n_extra - 1)];
-          }
-#pragma unroll
-          for (int e = 0; e < SCAN_PER; ++e) {
-            const int x = x0 + e * NT + tid;
-            if (x < n_extra && v[e] == -1 && extra_slot(x) < mine) mine = extra_slot(x);
-          }
-        }
-        if (mine < g.n_cmp) atomicMin(&first_neg[item_par], mine);
-      }
-      // block-table words (compiler-visible loads with in-bounds addresses)
-#pragma unroll
-      for (int e = 0; e < PER; ++e) {
-        const int r = e * NT + tid;
-        const int pos = c0 + r;
-        const bool win = pos < g.n_win;
-        const int key = win ? g.win_lo + pos : cid[e];
-        const int bsz = win ? a.ori_block_size : a.cmp_block_size;
-        const int tlen = win ? a.ori_table_len : a.cmp_table_len;
-        const int32_t* tbl = win ? a.ori_block_table : a.cmp_block_table;
-        const int bi = key >= 0 ? key / bsz : 0;
-        const bool ok = r < clen && tok_ok && key >= 0 && bi < tlen && (win || cid[e] < g.thr);
-        const int t = (tbl != nullptr) ? tbl[(size_t)b * tlen + (bi < tlen ? bi : tlen - 1)] : -1;
-        tab[e] = ok ? t : -1;
-      }
-      // every load so far (table words, query fragment) has landed, as the compiler sees it
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0) expcnt(7) lgkmcnt(15)
-      if (c0 == p_lo) m_run = seed_m();
-      if constexpr (QK8) {
-        quantize_q(qf, q8, sq);
-      }
-      if (stop_pending) {
-        __syncthreads();  // every thread's atomicMin is in
-        cmp_stop = min(first_neg[item_par], g.n_cmp);
-        if (tid == 0) first_neg[item_par ^ 1] = INT32_MAX;  // the next scan's slot
-        item_par ^= 1;
-        stop_pending = false;
-      }
-#pragma unroll
-      for (int e = 0; e < PER; ++e) {
-        const int r = e * NT + tid;
-        const int pos = c0 + r;
-        uint32_t id = ROW_INVALID;
-        const int phys = tab[e];
-        if (r < clen && tok_ok && phys >= 0) {
-          if (pos < g.n_win) {
-            if (phys < a.ori_block_num)
-              id = (uint32_t)(phys * a.ori_block_size + (g.win_lo + pos) % a.ori_block_size);
-          } else if (phys < a.cmp_block_num && (!scan3 || pos - g.n_win < cmp_stop)) {
-            id = (uint32_t)(phys * a.cmp_block_size + cid[e] % a.cmp_block_size) | 0x80000000u;
-          }
-        }
-        rowid[r] = id;  // masked rows are read from the zero row
-        const unsigned long long bal = __ballot(id != ROW_INVALID);
-        if (lane == 0) {
-          tmask[(r - lane) / TILE] = (uint32_t)bal;
-          tmask[(r - lane) / TILE + 1] = (uint32_t)(bal >> 32);
-        }
-      }
-      __syncthreads();
+      // ---- positions -> cache rows (bit 31: compressed cache) ----
+      res.template chunk<NT, RCH, RCH / NT + 4>(a, c0, clen, tid, rowid, tmask, first_neg, item_par, [&] {
+        if (c0 == p_lo) m_run = seed_m();
+        if constexpr (QK8) quantize_q(qf, q8, sq);
+      });
 
       // ---- DMA issue for one tile into one ring stage ----
       // main part: wave w fills rows w, w + NW, ...; one 1 KB row per instruction
@@ -2233,13 +2219,15 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
     // ---- epilogue: the item's rows go out through LDS (the ring is free), so
     // every store instruction writes whole rows ----
     {
+      const KernelArgs a = fresh_args();
+      int w_e = w;  // (the rows' addresses are formed here, not before the item loop)
+      asm volatile("" : "+s"(w_e));
       unsigned char* stg = kv_lds;
       const int nh = min(MB, a.num_heads - hb * MB);  // heads of this item
-      int tid_e = tid, hl_e = hp, dv_e = wq * DVQ + 4 * hl;
-      asm volatile("" : "+v"(tid_e), "+v"(hl_e), "+v"(dv_e));
+      int lane_e = lane, hl_e = hp, dv_e = wq * DVQ + 4 * hl;
+      asm volatile("" : "+v"(lane_e), "+v"(hl_e), "+v"(dv_e));
       if (!partial) {
         constexpr int SROW = DV * 2 + 16;  // staging row stride (bytes; 16-byte aligned rows)
-        constexpr int CPR = DV * 2 / 16;   // 16-byte chunks per row
         static_assert(MB * SROW <= NSTG * STAGE_BYTES, "output staging");
         const float inv = 1.0f / l_run;
 #pragma unroll
@@ -2256,10 +2244,9 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
         __syncthreads();
         if (tok_ok) {
           char* obase = (char*)((T*)a.out + ((size_t)tok * a.num_heads + hb * MB) * DV);
-          for (int c = tid_e; c < nh * CPR; c += NT) {
-            const int h = c / CPR, c16 = c - h * CPR;
-            *(i16x8*)(obase + (size_t)h * DV * 2 + c16 * 16) = *(const i16x8*)(stg + h * SROW + c16 * 16);
-          }
+          rows_out<MB, NW, SROW>(stg, nh, w_e, lane_e, [&](int h, i32x4 v) {
+            *(i32x4*)(obase + h * DV * 2 + 16 * lane_e) = v;
+          });
           if (wq == 0 && hl == 0 && head_p_ok)
             a.lse[(size_t)tok * a.num_heads + hb * MB + hl_e] = (m_fin + __log2f(l_run)) * LN2;
         }
@@ -2267,7 +2254,6 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
         // fp16 partials (acc / l, scaled): the row max over the four dv quarters
         // (lanes l, l ^ 32 of waves wq = 0..3) picks the scale; rows staged whole
         constexpr int SROW = DV * 2 + 16;  // staging row stride (bytes), as for the outputs
-        constexpr int CPR = DV * 2 / 16;   // 16-byte chunks per row
         static_assert(MB * SROW + 4 * MB * 4 <= NSTG * STAGE_BYTES, "partial staging");
         float* rmax = (float*)(stg + MB * SROW);
         const bool empty = !(l_run > 0.0f);
@@ -2296,10 +2282,9 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const SasAttnArgs a) {
           }
         __syncthreads();
         char* wbase = (char*)a.workspace + (size_t)slot * MB * DV * 2;
-        for (int c = tid_e; c < nh * CPR; c += NT) {
-          const int h = c / CPR, c16 = c - h * CPR;
-          *(i16x8*)(wbase + (size_t)h * DV * 2 + c16 * 16) = *(const i16x8*)(stg + h * SROW + c16 * 16);
-        }
+        rows_out<MB, NW, SROW>(stg, nh, w_e, lane_e, [&](int h, i32x4 v) {
+          *(i32x4*)(wbase + h * DV * 2 + 16 * lane_e) = v;
+        });
         if (wq == 0 && hl == 0 && head_p_ok) {
           float* wl = partial_lse(a, MB, DV);
           wl[(size_t)slot * MB + hl_e] = empty ? -INFINITY : (m_fin + __log2f(l_run)) * LN2;
@@ -2515,7 +2500,12 @@ static bool row_pairs_ok(const SasAttnArgs& a) {
 }
 
 template <int DQK, int NHG, typename T, int KVF>
-static hipError_t launch_attn(const SasAttnArgs& a, hipStream_t st) {
+static hipError_t launch_attn(const SasAttnArgs& args, hipStream_t st) {
+  KernelArgs a;
+  (SasAttnArgs&)a = args;
+  a.ori_bs = FastDiv::of(a.ori_block_size);
+  a.cmp_bs = a.scenario >= 2 ? FastDiv::of(a.cmp_block_size) : a.ori_bs;
+  a.ratio = a.scenario >= 2 ? FastDiv::of(a.cmp_ratio) : a.ori_bs;
   const int phases = (a.phases & 3) == 0 ? 3 : (a.phases & 3);
   if (phases & 1) {
     const int per_xcd = (a.num_fa + 7) / 8;
@@ -2565,7 +2555,7 @@ static hipError_t launch_attn(const SasAttnArgs& a, hipStream_t st) {
     const int groups = (a.m_base + MERGE_HPB - 1) / MERGE_HPB;  // head groups per task (upper bound)
     const int tasks = dev ? (a.num_fa < 256 ? a.num_fa : 256) : a.num_fd;  // columns; tasks strided
     const int cols = (tasks + 7) / 8 * 8;  // a multiple of the 8 XCDs
-    hipLaunchKernelGGL((merge_kernel<512, T>), dim3(cols, groups), dim3(MERGE_THREADS), 0, st, a);
+    hipLaunchKernelGGL((merge_kernel<512, T>), dim3(cols, groups), dim3(MERGE_THREADS), 0, st, args);
     return hipGetLastError();
   }
   return hipSuccess;

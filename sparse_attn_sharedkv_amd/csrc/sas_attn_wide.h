@@ -95,7 +95,7 @@ __device__ inline int wide_rope1(int l) {
 __device__ inline int wide_v(int l) { return wide_row_base(4 * (l >> 4) + ((l & 15) >> 2)) + 8 * (l & 3); }
 
 template <int DQK, int DV, typename T, int KVF = SAS_KV_NATIVE, bool PAIR = false, bool QK8 = false>
-__global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
+__global__ __launch_bounds__(512) void wide_kernel(const KernelArgs a) {
   constexpr int NW = 8;                  // waves per workgroup
   constexpr int MB = 128;                // query heads per workgroup (columns of Sᵀ)
   // PAIR: items of 64 heads (at most 64 heads, one head block), two consecutive
@@ -162,6 +162,18 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
   const int gsel = PAIR ? (w >> 2) : 0;    // row pairs: which of the two rows
   const int hlocal = PAIR ? srow & 63 : srow;  // head within the item's m-block
   const bool has_rope = ROPE && w < NROPE; // this wave issues rope DMA instruction w
+  // With at most 64 batches, every batch's lengths and query offset sit in one
+  // lane each, loaded at the start beside the metadata row; otherwise they are
+  // scalar loads per item.
+  const QRows qrows(a);
+  const bool lens_in_lanes = a.batch <= 64;
+  int lane_aq = 0, lane_kv = 0, lane_qp = 0;
+  if (lens_in_lanes) {
+    const int lb = lane < a.batch ? lane : a.batch - 1;
+    lane_aq = qrows.rows[lb];
+    lane_kv = a.seqused_kv[lb];
+    lane_qp = qrows.first[lb];
+  }
   int s2b = a.s2_base;
   int nfa = a.num_fa;
   if (a.num_fd == SAS_SCHED_DEVICE) {
@@ -180,7 +192,7 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
   if (fa[0] == 0) return;
   // where the whole schedule ends (loaded beside this row's cursors)
   const int32_t* fa_last = a.metadata + (nfa - 1) * SAS_FA_METADATA_SIZE;
-  const int last_b = fa_last[4] < a.batch ? fa_last[4] : a.batch;
+  const int last_b = fa_last[4] < 0 ? 0 : (fa_last[4] < a.batch ? fa_last[4] : a.batch);
   const int last_m = fa_last[4] < a.batch ? fa_last[5] : 0;
   int b = fa[1], m = fa[2];
   const int j_start = fa[3];
@@ -196,18 +208,6 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
   const char* ori_kv = (const char*)a.ori_kv;
   const char* cmp_kv = (const char*)(a.cmp_kv ? a.cmp_kv : a.ori_kv);
   const float sc = a.softmax_scale * LOG2E;
-  // With at most 64 batches, every batch's lengths and query offset sit in one
-  // lane each, loaded at the start beside the metadata row; otherwise they are
-  // scalar loads per item.
-  const QRows qrows(a);
-  const bool lens_in_lanes = a.batch <= 64;
-  int lane_aq = 0, lane_kv = 0, lane_qp = 0;
-  if (lens_in_lanes) {
-    const int lb = lane < a.batch ? lane : a.batch - 1;
-    lane_aq = qrows.rows[lb];
-    lane_kv = a.seqused_kv[lb];
-    lane_qp = qrows.first[lb];
-  }
   if (tid < 2) first_neg[tid] = INT32_MAX;
   // piece index of the first item when it continues a split item
   const int cont_k = (merge_here && j_start > 0) ? continued_piece_index(a, fa_row, b, m, cscan) : 0;
@@ -221,11 +221,12 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
   int tok_lo = 0, tok_hi = a.total_tokens;
   if (qrows.cumulative) {
     tok_lo = ld_uniform(qrows.first);
-    tok_hi = ld_uniform(qrows.first + last_b) + last_m / ((a.num_heads + IMB - 1) / IMB);
+    tok_hi = ld_uniform(qrows.first + last_b) + (last_m >> ((a.num_heads + IMB - 1) / IMB - 1));
   }
   int item_par = 0;  // which first_neg slot the next top-k scan uses
   bool first_item = true;
-  const int hblocks = (a.num_heads + IMB - 1) / IMB;
+  const int hblocks = (a.num_heads + IMB - 1) / IMB;  // 1 or 2 (the launch's check of m_base)
+  const int hshift = hblocks - 1;
   auto batch_lens = [&](int bb, int& aq, int& akv, int& qp) {
     const int bc = bb < a.batch ? bb : a.batch - 1;
     if (lens_in_lanes) {
@@ -240,6 +241,7 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
     }
   };
   for (;;) {
+    const KernelArgs a = fresh_args();
     b = __builtin_amdgcn_readfirstlane(b);
     m = __builtin_amdgcn_readfirstlane(m);
     int act_q, act_kv, qpre;
@@ -252,14 +254,14 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
     }
     if (b >= a.batch || b > b_end || (b == b_end && m > s_end)) break;
     const bool is_end = (b == b_end && m == s_end);
-    const int s = m / hblocks;
+    const int s = m >> hshift;
     const int hb = m - s * hblocks;
     const int head = hb * IMB + hlocal;
     if (is_end && j_end == 0) break;
 
     const int tok = qpre + s;
     const bool partial = (first_item && j_start > 0) || is_end;
-    ItemGeom g = item_geom(act_q, act_kv, s, a.ori_win_left, a.scenario, a.cmp_ratio, a.topk);
+    ItemGeom g = item_geom_at(a, act_q, act_kv, s);
     // row pairs: the next row joins when neither row is a piece of a split item,
     // and g becomes the union of the two rows' lists (the window rows of row
     // s + 1 start at or after those of row s, and the two windows touch)
@@ -268,7 +270,7 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
     if constexpr (PAIR) {
       if (!partial && hblocks == 1 && a.scenario <= 2 && m + 1 < act_q &&
           !(b == b_end && m + 1 >= s_end)) {
-        gB = item_geom(act_q, act_kv, s + 1, a.ori_win_left, a.scenario, a.cmp_ratio, a.topk);
+        gB = item_geom_at(a, act_q, act_kv, s + 1);
         const int hiA = gA.win_lo + gA.n_win, hiB = gB.win_lo + gB.n_win;
         if (gA.n_win == 0 && gB.n_win == 0) {
           pair = true;
@@ -297,12 +299,9 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
       }
     }
     const int L = g.n_win + g.n_cmp;
-    const int nblk = (L + s2b - 1) / s2b;
     const int blo = first_item ? j_start : 0;
-    int bhi = is_end ? j_end : nblk;
-    if (bhi > nblk) bhi = nblk;
     const int p_lo = blo * s2b;
-    const int p_hi = bhi * s2b < L ? bhi * s2b : L;
+    const int p_hi = is_end && (int64_t)j_end * s2b < L ? j_end * s2b : L;
     const bool tok_ok = tok >= 0 && tok < a.total_tokens;
     const bool tok_ok_w = tok_w >= 0 && tok_w < a.total_tokens;
 
@@ -325,20 +324,7 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
     i32x8 q8[QK8 ? 4 : 1];
     float sq = 1.0f;
 
-    // ---- scenario 3: position of the first -1 among the scanned top-k slots ----
-    // (golden.py:48-53: the scan stops at the first -1). The first chunk's own
-    // top-k loads double as the scan of its range; the slots outside it are
-    // loaded in the same batch, and the block-table loads of the chunk are
-    // issued before the barrier that publishes the result (the -1 cut is
-    // applied when the row ids are packed). The two first_neg slots alternate
-    // between scans, so a slot is reset without a barrier of its own.
-    const int32_t* idx_row =
-        a.cmp_indices ? a.cmp_indices + (size_t)(tok_ok ? tok : 0) * a.topk : nullptr;
-    const bool scan3 = a.scenario == 3 && idx_row != nullptr && a.topk > 0;
-    const int jmax = (scan3 && p_hi > g.n_win) ? min(p_hi - g.n_win, g.n_cmp) : 0;
-    bool stop_pending = jmax > 0;
-    int cmp_stop = g.n_cmp;
-
+    Resolver res(a, g, b, tok, tok_ok, p_hi);
     for (int c0 = p_lo; c0 < p_hi; c0 += RCH) {
       const int clen = (p_hi - c0) < RCH ? (p_hi - c0) : RCH;
       const int ntile = (clen + TILE - 1) / TILE;
@@ -360,121 +346,10 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
           qf[ks] = *(const i16x8*)(qrow + dim);
         }
       };
-      // ---- resolve positions -> cache rows (bit 31: compressed cache) ----
-      int cid[PER];
-      int tab[PER];
-      const int own_lo = max(c0 - g.n_win, 0);
-      const int own_hi = min(max(c0 + clen - g.n_win, own_lo), jmax);
-      const int n_extra = stop_pending ? jmax - (own_hi - own_lo) : 0;
-      constexpr int SCAN_PER = 6;  // first scan round: PER + SCAN_PER loads per thread
-      auto extra_slot = [&](int x) { return x < own_lo ? x : x + (own_hi - own_lo); };
-      int sv0[SCAN_PER];
-      if (scan3) {
-        // all loads issued and waited for in one asm statement (gather_dwords_wait)
-        const int32_t* src[PER + SCAN_PER];
-        int got[PER + SCAN_PER];
-#pragma unroll
-        for (int e = 0; e < PER; ++e) {
-          const int jj = c0 + e * NT + tid - g.n_win;
-          src[e] = idx_row + (jj < 0 ? 0 : (jj < a.topk ? jj : a.topk - 1));
-        }
-#pragma unroll
-        for (int e = 0; e < SCAN_PER; ++e) {
-          const int x = e * NT + tid;  // clamped into range; unused when n_extra == 0
-          const int xc = x < n_extra ? x : (n_extra > 0 ? n_extra - 1 : 0);
-          src[PER + e] = idx_row + (n_extra > 0 ? extra_slot(xc) : 0);
-        }
-        gather_dwords_wait(got, src);
-#pragma unroll
-        for (int e = 0; e < SCAN_PER; ++e) sv0[e] = got[PER + e];
-#pragma unroll
-        for (int e = 0; e < PER; ++e) {
-          const int r = e * NT + tid;
-          const int pos = c0 + r;
-          cid[e] = (r < clen && tok_ok && pos >= g.n_win) ? got[e] : -1;
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < PER; ++e) {
-          const int r = e * NT + tid;
-          const int pos = c0 + r;
-          cid[e] = (r < clen && tok_ok && pos >= g.n_win) ? pos - g.n_win : -1;
-        }
-      }
-      if (stop_pending) {
-        int mine = g.n_cmp;
-#pragma unroll
-        for (int e = 0; e < PER; ++e) {
-          const int jj = c0 + e * NT + tid - g.n_win;
-          if (jj >= 0 && jj < jmax && e * NT + tid < clen && cid[e] == -1 && jj < mine) mine = jj;
-        }
-#pragma unroll
-        for (int e = 0; e < SCAN_PER; ++e) {
-          const int x = e * NT + tid;
-          if (x < n_extra && sv0[e] == -1 && extra_slot(x) < mine) mine = extra_slot(x);
-        }
-        for (int x0 = NT * SCAN_PER; x0 < n_extra; x0 += NT * SCAN_PER) {  // beyond the first round
-          int v[SCAN_PER];
-#pragma unroll
-          for (int e = 0; e < SCAN_PER; ++e) {  // unconditional, clamped: all loads in flight at once
-            const int x = x0 + e * NT + tid;
-            v[e] = idx_row[extra_slot(x < n_extra ? x : n_extra - 1)];
-          }
-#pragma unroll
-          for (int e = 0; e < SCAN_PER; ++e) {
-            const int x = x0 + e * NT + tid;
-            if (x < n_extra && v[e] == -1 && extra_slot(x) < mine) mine = extra_slot(x);
-          }
-        }
-        if (mine < g.n_cmp) atomicMin(&first_neg[item_par], mine);
-      }
-      // block-table words (compiler-visible loads with in-bounds addresses)
-#pragma unroll
-      for (int e = 0; e < PER; ++e) {
-        const int r = e * NT + tid;
-        const int pos = c0 + r;
-        const bool win = pos < g.n_win;
-        const int key = win ? g.win_lo + pos : cid[e];
-        const int bsz = win ? a.ori_block_size : a.cmp_block_size;
-        const int tlen = win ? a.ori_table_len : a.cmp_table_len;
-        const int32_t* tbl = win ? a.ori_block_table : a.cmp_block_table;
-        const int bi = key >= 0 ? key / bsz : 0;
-        const bool ok = r < clen && tok_ok && key >= 0 && bi < tlen && (win || cid[e] < g.thr);
-        const int t = (tbl != nullptr) ? tbl[(size_t)b * tlen + (bi < tlen ? bi : tlen - 1)] : -1;
-        tab[e] = ok ? t : -1;
-      }
-      // every load so far (table words) has landed, as the compiler sees it
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0) expcnt(7) lgkmcnt(15)
-      if (c0 == p_lo) m_run = seed_m();
-      if (stop_pending) {
-        __syncthreads();  // every thread's atomicMin is in
-        cmp_stop = min(first_neg[item_par], g.n_cmp);
-        if (tid == 0) first_neg[item_par ^ 1] = INT32_MAX;  // the next scan's slot
-        item_par ^= 1;
-        stop_pending = false;
-      }
-#pragma unroll
-      for (int e = 0; e < PER; ++e) {
-        const int r = e * NT + tid;
-        const int pos = c0 + r;
-        uint32_t id = ROW_INVALID;
-        const int phys = tab[e];
-        if (r < clen && tok_ok && phys >= 0) {
-          if (pos < g.n_win) {
-            if (phys < a.ori_block_num)
-              id = (uint32_t)(phys * a.ori_block_size + (g.win_lo + pos) % a.ori_block_size);
-          } else if (phys < a.cmp_block_num && (!scan3 || pos - g.n_win < cmp_stop)) {
-            id = (uint32_t)(phys * a.cmp_block_size + cid[e] % a.cmp_block_size) | 0x80000000u;
-          }
-        }
-        rowid[r] = id;  // masked rows are read from the zero row
-        const unsigned long long bal = __ballot(id != ROW_INVALID);
-        if (lane == 0) {
-          tmask[(r - lane) / TILE] = (uint32_t)bal;
-          tmask[(r - lane) / TILE + 1] = (uint32_t)(bal >> 32);
-        }
-      }
-      __syncthreads();
+      // ---- positions -> cache rows (bit 31: compressed cache) ----
+      res.template chunk<NT, RCH, 8>(a, c0, clen, tid, rowid, tmask, first_neg, item_par, [&] {
+        if (c0 == p_lo) m_run = seed_m();
+      });
 
       // ---- DMA issue for one tile into one ring stage ----
       // main part: wave w fills rows w + 8 j (j < 4), one 1 KB row per instruction;
@@ -914,12 +789,14 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
     // every store instruction writes whole rows ----
     __syncthreads();  // (an item without rows: the previous item's staged rows are read out)
     {
+      const KernelArgs a = fresh_args();
+      int w_e = w;  // (the rows' addresses are formed here, not before the item loop)
+      asm volatile("" : "+s"(w_e));
       unsigned char* stg = kv_lds;
       const int nh = min(IMB, a.num_heads - hb * IMB);  // heads of this item
       constexpr int SROW = DV * 2 + 16;  // staging row stride (bytes; 16-byte aligned rows)
-      constexpr int CPR = DV * 2 / 16;   // 16-byte chunks per row
-      int tid_e = tid, hl_e = srow, dv_e = 4 * g4;
-      asm volatile("" : "+v"(tid_e), "+v"(hl_e), "+v"(dv_e));
+      int lane_e = lane, hl_e = srow, dv_e = 4 * g4;
+      asm volatile("" : "+v"(lane_e), "+v"(hl_e), "+v"(dv_e));
       if (!partial) {
         const float inv = 1.0f / l_run;
 #pragma unroll
@@ -933,18 +810,15 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
           if constexpr (PAIR) {
             // staging row h: row s + h / 64, head h % 64
             char* obase = (char*)((T*)a.out + (size_t)tok * a.num_heads * DV);
-            for (int c = tid_e; c < (pair ? 2 : 1) * 64 * CPR; c += NT) {
-              const int h = c / CPR, c16 = c - h * CPR;
+            rows_out<MB, NW, SROW>(stg, pair ? 128 : 64, w_e, lane_e, [&](int h, i32x4 v) {
               if ((h & 63) < a.num_heads && tok + (h >> 6) < a.total_tokens)
-                *(i16x8*)(obase + ((size_t)(h >> 6) * a.num_heads + (h & 63)) * DV * 2 + c16 * 16) =
-                    *(const i16x8*)(stg + h * SROW + c16 * 16);
-            }
+                *(i32x4*)(obase + ((h >> 6) * a.num_heads + (h & 63)) * DV * 2 + 16 * lane_e) = v;
+            });
           } else {
             char* obase = (char*)((T*)a.out + ((size_t)tok * a.num_heads + hb * MB) * DV);
-            for (int c = tid_e; c < nh * CPR; c += NT) {
-              const int h = c / CPR, c16 = c - h * CPR;
-              *(i16x8*)(obase + (size_t)h * DV * 2 + c16 * 16) = *(const i16x8*)(stg + h * SROW + c16 * 16);
-            }
+            rows_out<MB, NW, SROW>(stg, nh, w_e, lane_e, [&](int h, i32x4 v) {
+              *(i32x4*)(obase + h * DV * 2 + 16 * lane_e) = v;
+            });
           }
           if (g4 == 0 && head_ok && tok_ok_w)
             a.lse[(size_t)tok_w * a.num_heads + head] = (m_run + __log2f(l_run)) * LN2;
@@ -983,11 +857,9 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
           // read by another workgroup in this launch: agent-coherent stores
           const __amdgpu_buffer_rsrc_t rs = partial_rsrc(a, IMB, DV);
           const uint32_t base = (uint32_t)slot * IMB * DV * 2;
-          for (int c = tid_e; c < nh * CPR; c += NT) {
-            const int h = c / CPR, c16 = c - h * CPR;
-            partial_store16(rs, base + (uint32_t)(h * DV * 2 + c16 * 16),
-                            *(const i32x4*)(stg + h * SROW + c16 * 16));
-          }
+          rows_out<IMB, NW, SROW>(stg, nh, w_e, lane_e, [&](int h, i32x4 v) {
+            partial_store16(rs, base + (uint32_t)(h * DV * 2 + 16 * lane_e), v);
+          });
           if (g4 == 0 && head_ok) {
             const uint32_t lo = (uint32_t)a.num_partial_slots * IMB * DV * 2;
             partial_store4(rs, lo + ((uint32_t)slot * IMB + hl_e) * 4, lse_piece);
@@ -996,11 +868,9 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
           }
         } else {
           char* wbase = (char*)a.workspace + (size_t)slot * IMB * DV * 2;
-          for (int c = tid_e; c < nh * CPR; c += NT) {
-            const int h = c / CPR, c16 = c - h * CPR;
-            *(i16x8*)(wbase + (size_t)h * DV * 2 + c16 * 16) =
-                *(const i16x8*)(stg + h * SROW + c16 * 16);
-          }
+          rows_out<IMB, NW, SROW>(stg, nh, w_e, lane_e, [&](int h, i32x4 v) {
+            *(i32x4*)(wbase + h * DV * 2 + 16 * lane_e) = v;
+          });
           if (g4 == 0 && head_ok) {
             float* wl = partial_lse(a, IMB, DV);
             wl[(size_t)slot * IMB + hl_e] = lse_piece;
@@ -1011,8 +881,10 @@ __global__ __launch_bounds__(512) void wide_kernel(const SasAttnArgs a) {
     }
     if (partial && merge_here) {
       // the piece that completes the item merges it (bit-identical to merge_kernel)
+      const KernelArgs a = fresh_args();
       const int slot0 = (first_item && j_start > 0) ? slot - cont_k : slot;
       if (slot0 >= 0 && slot < a.num_partial_slots && slot0 < SAS_MERGE_SYNC_WORDS) {
+        const int nblk = (L + s2b - 1) / s2b, bhi = p_hi < L ? j_end : nblk;
         const int npc = split_arrive(a, slot0, slot, bhi - blo, bhi == nblk, nblk, &merge_word);
         if (npc > 0) merge_item_here<DV, T, IMB, NW>(a, tok, hb, slot0, npc);
       }
