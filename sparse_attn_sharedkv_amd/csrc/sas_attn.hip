@@ -305,6 +305,20 @@ __device__ __forceinline__ KernelArgs fresh_args() {
 #pragma unroll
   for (int i = 0; i < (int)(sizeof(KernelArgs) / 4); ++i) words[i] = p[i];
   __builtin_memcpy(&a, words, sizeof(a));
+  // device memory, said so: the compiler takes it for granted of pointers in the
+  // launch's own arguments only, and would access these with flat instructions (which
+  // return out of order, so each wait for one is a wait for every access in flight,
+  // the row DMAs included)
+  auto dev = [](auto*& q) {
+    typedef __typeof__(*q) SAS_GLOBAL* global_p;
+    q = (__typeof__(q + 0))(global_p)(uintptr_t)q;
+  };
+  auto devv = [](const void*& q) { q = (const void*)(const char*)(const char SAS_GLOBAL*)(uintptr_t)q; };
+  devv(a.q), devv(a.ori_kv), devv(a.cmp_kv);
+  dev(a.ori_block_table), dev(a.cmp_block_table), dev(a.cmp_indices), dev(a.q_prefix);
+  dev(a.act_q_lens), dev(a.seqused_kv), dev(a.sinks), dev(a.metadata), dev(a.lse);
+  dev(a.workspace), dev(a.merge_sync);
+  a.out = (void*)(char*)(char SAS_GLOBAL*)(uintptr_t)a.out;
   return a;
 }
 
