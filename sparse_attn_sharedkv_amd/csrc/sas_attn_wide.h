@@ -439,7 +439,6 @@ __global__ __launch_bounds__(512) void wide_kernel(const KernelArgs a) {
       // consecutive 16-byte chunks: no bank conflicts); the first 256 threads copy
       // the 32 x 8 rope chunks.
       auto convert_row = [&](int tile, int k) {
-        typedef int i32x2 __attribute__((ext_vector_type(2)));
         const int l = lane_id_here();  // (recomputed here: no offset stays live across the loop)
         const uint32_t st = kv_base + (uint32_t)((tile % 2) * STAGE_BYTES);
         const int r = w + NW * k;
@@ -785,8 +784,8 @@ __global__ __launch_bounds__(512) void wide_kernel(const KernelArgs a) {
       l_run = wave_sum_pair(__uint_as_float(r1[0]) + __uint_as_float(r1[1]));
     }
 
-    // ---- epilogue: the item's rows go out through LDS (the ring is free), so
-    // every store instruction writes whole rows ----
+    // ---- epilogue (pieces of split items go out through LDS, the ring being free, so
+    // every store instruction writes whole rows) ----
     __syncthreads();  // (an item without rows: the previous item's staged rows are read out)
     {
       const KernelArgs a = fresh_args();
@@ -798,30 +797,31 @@ __global__ __launch_bounds__(512) void wide_kernel(const KernelArgs a) {
       int lane_e = lane, hl_e = srow, dv_e = 4 * g4;
       asm volatile("" : "+v"(lane_e), "+v"(hl_e), "+v"(dv_e));
       if (!partial) {
+        // straight from the registers: lanes l and l ^ 16 trade halves of two dv blocks,
+        // so each holds 16 bytes of its head's row (head r16, dv 16 (d + g4 % 2) +
+        // 8 (g4 / 2) .. + 7) and a store instruction writes 64-byte pieces of 16 rows,
+        // whose other halves follow in the next. Through LDS, for whole 1 KB rows a
+        // store, this took a barrier and an LDS round trip more (us a kernel: 8K prefill,
+        // window / dense, 389 -> 384 / 412 -> 402, two rows a sequence 107.7 -> 106.0, fp8
+        // rows of 128 sequences, with fewer spills, 114.2 -> 111.6)
         const float inv = 1.0f / l_run;
+        if (tok_ok_w && head_ok) {
+          const size_t row = (size_t)tok_w * a.num_heads + head;
+          char* orow = (char*)a.out + row * DV * 2 + 32 * (g4 & 1) + 16 * (g4 >> 1);
 #pragma unroll
-        for (int d = 0; d < NDV; ++d) {
-          const i16x4 v = {Ops::from_f32(acc[d][0] * inv), Ops::from_f32(acc[d][1] * inv),
-                           Ops::from_f32(acc[d][2] * inv), Ops::from_f32(acc[d][3] * inv)};
-          *(i16x4*)(stg + hl_e * SROW + (16 * d + dv_e) * 2) = v;
-        }
-        __syncthreads();
-        if (tok_ok) {
-          if constexpr (PAIR) {
-            // staging row h: row s + h / 64, head h % 64
-            char* obase = (char*)((T*)a.out + (size_t)tok * a.num_heads * DV);
-            rows_out<MB, NW, SROW>(stg, pair ? 128 : 64, w_e, lane_e, [&](int h, i32x4 v) {
-              if ((h & 63) < a.num_heads && tok + (h >> 6) < a.total_tokens)
-                *(i32x4*)(obase + ((h >> 6) * a.num_heads + (h & 63)) * DV * 2 + 16 * lane_e) = v;
-            });
-          } else {
-            char* obase = (char*)((T*)a.out + ((size_t)tok * a.num_heads + hb * MB) * DV);
-            rows_out<MB, NW, SROW>(stg, nh, w_e, lane_e, [&](int h, i32x4 v) {
-              *(i32x4*)(obase + h * DV * 2 + 16 * lane_e) = v;
-            });
+          for (int d = 0; d < NDV; d += 2) {
+            i32x2 x[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+              const i16x4 v = {Ops::from_f32(acc[d + e][0] * inv), Ops::from_f32(acc[d + e][1] * inv),
+                               Ops::from_f32(acc[d + e][2] * inv), Ops::from_f32(acc[d + e][3] * inv)};
+              x[e] = __builtin_bit_cast(i32x2, v);
+            }
+            const auto lo = __builtin_amdgcn_permlane16_swap(x[0][0], x[1][0], false, false);
+            const auto hi = __builtin_amdgcn_permlane16_swap(x[0][1], x[1][1], false, false);
+            *(i32x4*)(orow + 32 * d) = (i32x4){(int)lo[0], (int)hi[0], (int)lo[1], (int)hi[1]};
           }
-          if (g4 == 0 && head_ok && tok_ok_w)
-            a.lse[(size_t)tok_w * a.num_heads + head] = (m_run + __log2f(l_run)) * LN2;
+          if (g4 == 0) a.lse[row] = (m_run + __log2f(l_run)) * LN2;
         }
       } else if (slot >= 0 && slot < a.num_partial_slots && a.workspace) {
         // (row pairs: a piece of a split item is never paired, so its heads are
