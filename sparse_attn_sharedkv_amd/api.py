@@ -24,6 +24,7 @@ for launch failures. Everything is checked on the host before any launch.
 
 from __future__ import annotations
 
+import collections
 import ctypes
 import functools
 import threading
@@ -106,6 +107,39 @@ def _cached_schedule(act_q: tuple, act_kv: tuple, num_heads: int, ori_win_left: 
     return md, _max_pieces(md)
 
 
+# Between a host-scheduled call's lengths arriving and its launch the GPU waits, so
+# prepare() reads the lengths back behind the rest of its work, and the cached host
+# schedules are kept on the GPU they were used on, by their inputs: a call whose
+# lengths give a known one does not copy its 64 KB again. Calls of 8192 query rows in
+# a row, 64 heads, on one MI355X: window-only 449 -> 409 us, dense pool 482 -> 426,
+# top-k 1143 -> 1078, with the kernels' own 384, 402 and 1069. (The on-device
+# scheduler instead was slower: such schedules, of more than ~4000 items, are rebuilt
+# on each call, 120 us.) An entry is complete before it is handed out, so any stream
+# may read it; a use on another stream than its own is recorded, so that an evicted
+# one is not given out again under a kernel that still reads it.
+_GPU_SCHEDULES: "collections.OrderedDict" = collections.OrderedDict()
+_GPU_SCHEDULES_MAX = 64
+_GPU_SCHEDULES_LOCK = threading.Lock()
+
+
+def _schedule_on(dev: torch.device, key: tuple, md: torch.Tensor) -> torch.Tensor:
+    st = torch.cuda.current_stream(dev)
+    with _GPU_SCHEDULES_LOCK:
+        hit = _GPU_SCHEDULES.get((dev, key))
+        if hit is not None:
+            _GPU_SCHEDULES.move_to_end((dev, key))
+    if hit is None:
+        hit = (md.to(dev), st.cuda_stream)
+        st.synchronize()
+        with _GPU_SCHEDULES_LOCK:
+            _GPU_SCHEDULES[(dev, key)] = hit
+            while len(_GPU_SCHEDULES) > _GPU_SCHEDULES_MAX:
+                _GPU_SCHEDULES.popitem(last=False)
+    if hit[1] != st.cuda_stream:
+        hit[0].record_stream(st)
+    return hit[0]
+
+
 # Schedules built by the on-device scheduler for calls without ``metadata``: one
 # library-owned buffer per (device, stream), written only by that scheduler on
 # that stream, so an unchanged schedule is kept instead of rebuilt. Calls on one
@@ -170,7 +204,19 @@ def _merge_sync_buffer(dev: torch.device, st: torch.cuda.Stream) -> torch.Tensor
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    return t.data_ptr() if t is not None else None
+
+
+def _read_back(ts):
+    """int32 tensors on one GPU on their way to the host: ``(pinned words, event)``."""
+    host = torch.empty(sum(t.numel() for t in ts), dtype=torch.int32, pin_memory=True)
+    at = 0
+    for t in ts:
+        host[at:at + t.numel()].copy_(t, non_blocking=True)
+        at += t.numel()
+    done = torch.cuda.Event()
+    done.record(torch.cuda.current_stream(ts[0].device))
+    return host, done
 
 
 def prepare(q: torch.Tensor, *, ori_kv: torch.Tensor, cmp_kv: Optional[torch.Tensor] = None,
@@ -231,13 +277,22 @@ def prepare(q: torch.Tensor, *, ori_kv: torch.Tensor, cmp_kv: Optional[torch.Ten
 
     # ---- flatten Q / indices to [total_tokens, ...] (api.py:208-240) ----
     cu_host = None
+    # lengths read back for a host schedule: late, behind the rest of the preparation
+    late = (_stream_schedule and metadata is None and not use_dev and q.is_cuda
+            and seqused_kv.is_cuda and seqused_kv.dim() == 1 and seqused_kv.numel() > 0
+            and not torch.cuda.is_current_stream_capturing())
     if layout_q == "TND":
         assert cu_seqlens_q is not None, "cu_seqlens_q is required for TND"
         if q.dim() != 3:
             raise ValueError(f"TND q must be [T, N1, D], got {tuple(q.shape)}")
         t1, n1, d = q.shape
         total = t1
-        if use_dev:  # lengths stay on the GPU; rows past cu_seqlens_q[-1] are zero-filled
+        # the launch takes cu_seqlens_q itself (QLENS_CUMULATIVE below): the host needs
+        # it for the schedule only
+        late = late and t1 > 0 and cu_seqlens_q.dim() == 1 and cu_seqlens_q.numel() > 1 \
+            and cu_seqlens_q.is_cuda
+        if use_dev or late:
+            # lengths stay on the GPU; rows past cu_seqlens_q[-1] are zero-filled
             nb = cu_seqlens_q.numel() - 1
             act_q = prefix = None
             padded = True
@@ -255,6 +310,7 @@ def prepare(q: torch.Tensor, *, ori_kv: torch.Tensor, cmp_kv: Optional[torch.Ten
         prefix = [i * s_max for i in range(nb)]
         act_q = [s_max] * nb
         padded = False
+        late = late and cu_seqlens_q is None and total > 0
         if cu_seqlens_q is not None and use_dev:
             act_q = None
             padded = True
@@ -337,7 +393,7 @@ def prepare(q: torch.Tensor, *, ori_kv: torch.Tensor, cmp_kv: Optional[torch.Ten
     if dev.type != "cuda":
         raise RuntimeError("sparse_attn_sharedkv runs on a ROCm GPU; q is on " + str(dev))
 
-    # ---- schedule (api.py:335-366) ----
+    # ---- query rows and lengths ----
     i32 = torch.int32
     seqused = seqused_kv.to(device=dev, dtype=i32).contiguous()
     # Callers that launch right after preparing hand the kernels cu_seqlens_q itself,
@@ -352,6 +408,48 @@ def prepare(q: torch.Tensor, *, ori_kv: torch.Tensor, cmp_kv: Optional[torch.Ten
         elif cu_seqlens_q is None:
             q_lens = _lib.QLENS_UNIFORM
             q_prefix = None
+    # ---- device tensors ----
+    q_flat = q.reshape(total, n1, d).contiguous()
+    ori_kv_d = ori_kv.contiguous()
+    ori_bt = ori_block_table.to(device=dev, dtype=i32).contiguous()
+    cmp_kv_d = cmp_kv.contiguous() if cmp_kv is not None else None
+    cmp_bt = cmp_block_table.to(device=dev, dtype=i32).contiguous() if cmp_kv is not None else None
+    idx_d = idx_flat.to(device=dev, dtype=i32).contiguous() if idx_flat is not None else None
+    if not use_dev and q_lens == _lib.QLENS_ARRAYS:
+        q_prefix = torch.tensor(prefix, dtype=i32).to(dev, non_blocking=True)
+        act_q_d = torch.tensor(act_q, dtype=i32).to(dev, non_blocking=True)
+    sinks_d = sinks.to(device=dev, dtype=torch.float32).contiguous()
+    if sinks_d.numel() != n1:
+        raise ValueError(f"sinks must have N1={n1} entries")
+    alloc = torch.zeros if padded else torch.empty
+    out = alloc((total, n1, dv), dtype=dtype, device=dev)
+    lse = alloc((total, n1), dtype=torch.float32, device=dev)
+    for t in (q_flat, ori_kv_d, cmp_kv_d):
+        if t is not None and t.device != dev:
+            raise ValueError("all tensors must be on q's device")
+
+    lens = None
+    if late:
+        lens = _read_back([cu_d, seqused] if layout_q == "TND" else [seqused])
+
+    a = _lib.SasAttnArgs()
+    a.q, a.ori_kv, a.ori_block_table = _ptr(q_flat), _ptr(ori_kv_d), _ptr(ori_bt)
+    a.cmp_kv, a.cmp_block_table, a.cmp_indices = _ptr(cmp_kv_d), _ptr(cmp_bt), _ptr(idx_d)
+    a.seqused_kv = _ptr(seqused)
+    a.sinks, a.out, a.lse = _ptr(sinks_d), _ptr(out), _ptr(lse)
+    a.batch, a.total_tokens, a.num_heads = nb, total, n1
+    a.head_dim, a.head_dim_v = d, dv
+    a.ori_block_num, a.ori_block_size, a.ori_table_len = (
+        ori_kv_d.shape[0], ori_kv_d.shape[1], ori_bt.shape[1])
+    if cmp_kv_d is not None:
+        a.cmp_block_num, a.cmp_block_size, a.cmp_table_len = (
+            cmp_kv_d.shape[0], cmp_kv_d.shape[1], cmp_bt.shape[1])
+    a.topk = int(k)
+    a.scenario, a.cmp_ratio, a.ori_win_left, a.dtype = scenario, cmp_ratio_eff, ori_win_left, dcode
+    a.softmax_scale = float(softmax_scale)
+    a.kv_format = kv_fmt
+
+    # ---- schedule (api.py:335-366) ----
     if use_dev:
         # per-batch query rows and first flat token, computed on the GPU
         if q_lens != _lib.QLENS_ARRAYS:
@@ -398,12 +496,20 @@ def prepare(q: torch.Tensor, *, ori_kv: torch.Tensor, cmp_kv: Optional[torch.Ten
         few_pieces = (int(core_num) <= MERGE_IN_KERNEL_MAX_PIECES * items
                       or most <= MERGE_IN_KERNEL_MAX_PIECES)
     elif metadata is None:
-        kv_host = tuple(int(x) for x in seqused_kv.to(torch.int32).cpu().tolist())
-        md, max_pieces = _cached_schedule(tuple(act_q), kv_host, int(n1), int(ori_win_left),
-                                          scenario, cmp_ratio_eff, int(k), int(core_num),
-                                          item64, m_base)
+        if lens is not None:  # everything else is ready: from here to the launch the GPU waits
+            lens[1].synchronize()
+            words = lens[0].tolist()
+            kv_host = tuple(words[-seqused.numel():])
+            if layout_q == "TND":
+                act_q = [b - a for a, b in zip(words[:nb], words[1:nb + 1])]
+        else:
+            kv_host = tuple(int(x) for x in seqused_kv.to(torch.int32).cpu().tolist())
+        key = (tuple(act_q), kv_host, int(n1), int(ori_win_left), scenario, cmp_ratio_eff, int(k),
+               int(core_num), item64, m_base)
+        md, max_pieces = _cached_schedule(*key)
         cfg = config_row(md)
-        metadata_dev = md.to(dev, non_blocking=True)
+        metadata_dev = (_schedule_on(dev, key, md) if lens is not None
+                        else md.to(dev, non_blocking=True))
         few_pieces = max_pieces <= MERGE_IN_KERNEL_MAX_PIECES
     else:
         metadata_dev = metadata.to(dev).to(torch.int32).reshape(SAS_META_SIZE).contiguous()
@@ -413,49 +519,13 @@ def prepare(q: torch.Tensor, *, ori_kv: torch.Tensor, cmp_kv: Optional[torch.Ten
         assert cfg["num_heads"] == n1 and m_base_valid(n1, item64, cfg["m_base"]), (
             "metadata was built for a different head count or cache row format "
             "(fp8 cache rows: sparse_attn_sharedkv_metadata(..., kv_cache_dtype='fp8_ds_mla'))")
-
-    # ---- device tensors ----
-    q_flat = q.reshape(total, n1, d).contiguous()
-    ori_kv_d = ori_kv.contiguous()
-    ori_bt = ori_block_table.to(device=dev, dtype=i32).contiguous()
-    cmp_kv_d = cmp_kv.contiguous() if cmp_kv is not None else None
-    cmp_bt = cmp_block_table.to(device=dev, dtype=i32).contiguous() if cmp_kv is not None else None
-    idx_d = idx_flat.to(device=dev, dtype=i32).contiguous() if idx_flat is not None else None
-    if not use_dev and q_lens == _lib.QLENS_ARRAYS:
-        q_prefix = torch.tensor(prefix, dtype=i32).to(dev, non_blocking=True)
-        act_q_d = torch.tensor(act_q, dtype=i32).to(dev, non_blocking=True)
-    sinks_d = sinks.to(device=dev, dtype=torch.float32).contiguous()
-    if sinks_d.numel() != n1:
-        raise ValueError(f"sinks must have N1={n1} entries")
-    alloc = torch.zeros if padded else torch.empty
-    out = alloc((total, n1, dv), dtype=dtype, device=dev)
-    lse = alloc((total, n1), dtype=torch.float32, device=dev)
     ws = None
     if cfg["num_fd"] > 0 or use_dev:
         nbytes = _lib.load().sas_workspace_bytes(cfg["num_partial_slots"], cfg["m_base"], dv)
         ws = torch.empty(nbytes // 4, dtype=torch.float32, device=dev)
 
-    for t in (q_flat, ori_kv_d, cmp_kv_d):
-        if t is not None and t.device != dev:
-            raise ValueError("all tensors must be on q's device")
-
-    a = _lib.SasAttnArgs()
-    a.q, a.ori_kv, a.ori_block_table = _ptr(q_flat), _ptr(ori_kv_d), _ptr(ori_bt)
-    a.cmp_kv, a.cmp_block_table, a.cmp_indices = _ptr(cmp_kv_d), _ptr(cmp_bt), _ptr(idx_d)
-    a.q_prefix, a.act_q_lens, a.seqused_kv = _ptr(q_prefix), _ptr(act_q_d), _ptr(seqused)
-    a.sinks, a.metadata = _ptr(sinks_d), _ptr(metadata_dev)
-    a.out, a.lse, a.workspace = _ptr(out), _ptr(lse), _ptr(ws)
-    a.batch, a.total_tokens, a.num_heads = nb, total, n1
-    a.head_dim, a.head_dim_v = d, dv
-    a.ori_block_num, a.ori_block_size, a.ori_table_len = (
-        ori_kv_d.shape[0], ori_kv_d.shape[1], ori_bt.shape[1])
-    if cmp_kv_d is not None:
-        a.cmp_block_num, a.cmp_block_size, a.cmp_table_len = (
-            cmp_kv_d.shape[0], cmp_kv_d.shape[1], cmp_bt.shape[1])
-    a.topk = int(k)
-    a.scenario, a.cmp_ratio, a.ori_win_left, a.dtype = scenario, cmp_ratio_eff, ori_win_left, dcode
-    a.softmax_scale = float(softmax_scale)
-    a.kv_format = kv_fmt
+    a.q_prefix, a.act_q_lens = _ptr(q_prefix), _ptr(act_q_d)
+    a.metadata, a.workspace = _ptr(metadata_dev), _ptr(ws)
     a.num_fa, a.num_fd = cfg["num_fa"], cfg["num_fd"]
     a.num_partial_slots, a.s2_base, a.m_base = (
         cfg["num_partial_slots"], cfg["s2_base"], cfg["m_base"])
