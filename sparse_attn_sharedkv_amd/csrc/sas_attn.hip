@@ -137,18 +137,24 @@ __device__ inline float wave_sum_pair(float v) {
 // Direct-to-LDS 16-byte loads: lane's data lands at M0 + lane * 16.
 // Issued through inline asm so the compiler does not serialise them against
 // unrelated LDS reads; completion is tracked by hand with s_waitcnt vmcnt.
-// An LDS DMA that reads M0 needs one wait state after the SALU write of M0
-// (the compiler's hazard pass cannot see inside the asm), hence the s_nop.
+// The compiler's hazard pass cannot see inside the asm, which therefore keeps two
+// rules itself: an LDS DMA needs one wait state after the SALU write of M0 it reads,
+// and a VMEM instruction five after a VALU write of an SGPR it reads. Row addresses
+// come from v_readlane (a VALU write), so the DMA takes a copy made by an s_mov_b64:
+// scalar instructions may read such an SGPR at once, and an SGPR written by one is
+// interlocked. The s_mov_b64 is M0's wait state, too.
 // Rows are fetched with the streaming cache policy (sc0 nt): each row is read
 // once per workgroup (the second 64-head m-block of a token reads it on the
 // same XCD shortly after), and the non-temporal fills shortened the stalls of
 // the DMA issue on every tile (measured about 3.5 us of 66 at B = 64, H = 128).
 __device__ inline void dma16_sbase(const void* sbase, uint32_t voff, uint32_t lds_base) {
+  uint64_t base;
   asm volatile(
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, %1 sc0 nt\n\t" ::"v"(voff),
-      "s"(sbase), "s"(lds_base)
+      "s_mov_b32 m0, %3\n\t"
+      "s_mov_b64 %0, %2\n\t"
+      "global_load_lds_dwordx4 %1, %0 sc0 nt\n\t"
+      : "=&s"(base)
+      : "v"(voff), "s"(sbase), "s"(lds_base)
       : "memory");
 }
 // dma16_sbase on the lanes of `lanes` only (lane i still writes lds_base + 16 i):
@@ -156,15 +162,15 @@ __device__ inline void dma16_sbase(const void* sbase, uint32_t voff, uint32_t ld
 // it change
 __device__ inline void dma16_sbase_lanes(const void* sbase, uint32_t voff, uint32_t lds_base,
                                          uint64_t lanes) {
-  uint64_t saved;
+  uint64_t saved, base;
   asm volatile(
       "s_mov_b64 %0, exec\n\t"
-      "s_mov_b64 exec, %4\n\t"
-      "s_mov_b32 m0, %3\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, %2 sc0 nt\n\t"
+      "s_mov_b64 exec, %5\n\t"
+      "s_mov_b32 m0, %4\n\t"
+      "s_mov_b64 %1, %3\n\t"
+      "global_load_lds_dwordx4 %2, %1 sc0 nt\n\t"
       "s_mov_b64 exec, %0\n\t"
-      : "=&s"(saved)
+      : "=&s"(saved), "=&s"(base)
       : "v"(voff), "s"(sbase), "s"(lds_base), "s"(lanes)
       : "memory");
 }
