@@ -208,14 +208,15 @@ typedef struct SasAttnArgs {
    * merges in a separate stage, metadata.py:925-954). NULL: the merge kernel runs after
    * the attention kernel, as in the reference. Otherwise SAS_MERGE_SYNC_WORDS arrival
    * counters (device memory, 8-byte aligned) that are zero before the call: each piece
-   * of a split item adds its block count to its item's counter after storing its
-   * partial, and the piece that completes the count merges the item's partials into
+   * of a split item counts itself in at its item's counter after storing its partial,
+   * and the piece that completes the schedule's count merges the item's partials into
    * out and lse at once, so the merge kernel is not launched (the merge phase enqueues
-   * nothing). The completing piece returns the counter to zero, so a buffer zeroed once
-   * stays usable; calls that may overlap (other streams, graphs replayed concurrently)
-   * need distinct buffers. Results are bit-identical to the merge kernel's. Native
-   * cache rows only (not with SAS_PHASE_PIPELINED); fp8 rows ignore it and run the
-   * merge kernel. */
+   * nothing). The completing piece returns the counter to zero, also when the lengths
+   * are not those of the schedule any more, so a buffer zeroed once stays usable; calls
+   * that may overlap (other streams, graphs replayed concurrently) need distinct
+   * buffers. Results are bit-identical to the merge kernel's. Native cache rows (not
+   * with SAS_PHASE_PIPELINED) and fp8 rows in 128-head items; fp8 rows in smaller items
+   * ignore it and run the merge kernel. */
   uint64_t* merge_sync;
 } SasAttnArgs;
 

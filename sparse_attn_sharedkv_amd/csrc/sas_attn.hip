@@ -616,32 +616,46 @@ __device__ inline void partial_store4(__amdgpu_buffer_rsrc_t r, uint32_t off, fl
   __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v), r, (int)off, 0, CPOL_SC1);
 }
 
-// Arrival of a piece whose partial every thread of the workgroup has stored
-// (with partial_store16 / partial_store4): adds the piece's blocks (low 32 bits)
-// and, from the item's final piece, the piece count (high 32 bits) to the item's
-// counter merge_sync[slot0]. Returns the piece count to the piece that completes
-// the item's blocks (it merges the item and has returned the counter to zero),
-// 0 to the others.
-__device__ inline int split_arrive(const SasAttnArgs& a, int slot0, int slot, int blocks,
-                                   bool final_piece, int nblk, int* lds_word) {
+// One thread counts a piece of the item in slots slot0, ... in at the item's counter
+// merge_sync[slot0]: pieces in the low 32 bits and, from the item's final piece (which
+// alone knows it), the piece count in the high ones. Returns the piece count to the
+// piece that completes it, 0 to the others, and then the counter is zero again. Pieces
+// are counted, not their blocks: every piece of the schedule counts itself in once
+// (split_settle), so a counter returns to zero whatever lengths a call finds.
+__device__ inline int split_count(const SasAttnArgs& a, int slot0, int slot, bool final_piece) {
+  const unsigned long long add =
+      1ull | (final_piece ? (unsigned long long)(uint32_t)(slot - slot0 + 1) << 32 : 0ull);
+  unsigned long long* c = (unsigned long long*)a.merge_sync + slot0;
+  const unsigned long long tot =
+      __hip_atomic_fetch_add(c, add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + add;
+  if ((uint32_t)tot != (uint32_t)(tot >> 32)) return 0;
+  __hip_atomic_store(c, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return (int)(tot >> 32);
+}
+__device__ inline bool split_slots_ok(const SasAttnArgs& a, int slot0, int slot) {
+  return slot0 >= 0 && slot < a.num_partial_slots && slot0 < SAS_MERGE_SYNC_WORDS;
+}
+// Arrival of a piece whose partial every thread of the workgroup has stored (with
+// partial_store16 / partial_store4); the piece that gets a count merges the item.
+__device__ inline int split_arrive(const SasAttnArgs& a, int slot0, int slot, bool final_piece,
+                                   int* lds_word) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's partial stores are done
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const unsigned long long add =
-        (unsigned long long)(uint32_t)blocks |
-        (final_piece ? (unsigned long long)(uint32_t)(slot - slot0 + 1) << 32 : 0ull);
-    unsigned long long* c = (unsigned long long*)a.merge_sync + slot0;
-    const unsigned long long tot =
-        __hip_atomic_fetch_add(c, add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + add;
-    int r = 0;
-    if ((uint32_t)tot == (uint32_t)nblk) {
-      r = (int)(tot >> 32);
-      __hip_atomic_store(c, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    *lds_word = r;
-  }
+  if (threadIdx.x == 0) *lds_word = split_count(a, slot0, slot, final_piece);
   __syncthreads();
   return *lds_word;
+}
+// After a workgroup's items: the pieces of its row whose items the call does not have
+// (fewer query rows than scheduled). `slot` is the next piece's; first: the row's first
+// piece, which continues an item (cont_k), is not counted in; last: its last is not.
+__device__ inline void split_settle(const SasAttnArgs& a, bool first, int cont_k, bool last, int slot) {
+  if (threadIdx.x != 0) return;
+  if (first) {
+    const int k = cont_k < 0 ? -cont_k : cont_k;
+    if (split_slots_ok(a, slot - k, slot)) split_count(a, slot - k, slot, cont_k > 0);
+    ++slot;
+  }
+  if (last && split_slots_ok(a, slot, slot)) split_count(a, slot, slot, false);
 }
 
 // Merge of split item (token tok, head block hb; pieces in slots slot0 ..
@@ -945,8 +959,18 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const KernelArgs a) {
   const char* cmp_kv = (const char*)(a.cmp_kv ? a.cmp_kv : a.ori_kv);
   const float sc = a.softmax_scale * LOG2E;
   if (tid < 2) first_neg[tid] = INT32_MAX;
-  // piece index of the first item when it continues a split item
-  const int cont_k = (merge_here && j_start > 0) ? continued_piece_index(a, fa_row, b, m, cscan) : 0;
+  // piece index of the first item when it continues a split item, negative when the
+  // item goes on in the next row (by the schedule, whatever the lengths are by now);
+  // last_owed: the row's last piece, of an item that begins here, is not counted in
+  int cont_k = 0;
+  bool last_owed = merge_here && j_end > 0;
+  if (merge_here && j_start > 0) {
+    cont_k = continued_piece_index(a, fa_row, b, m, cscan);
+    if (j_end > 0 && b == b_end && m == s_end) {
+      cont_k = -cont_k;
+      last_owed = false;
+    }
+  }
   __syncthreads();
 
   // Sinks of this lane's head in the (at most two) head blocks of an item,
@@ -1487,18 +1511,21 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const KernelArgs a) {
     if (partial && merge_here) {
       // the piece that completes the item merges it (bit-identical to merge_kernel)
       const KernelArgs a = fresh_args();
-      const int slot0 = (first_item && j_start > 0) ? slot - cont_k : slot;
-      if (slot0 >= 0 && slot < a.num_partial_slots && slot0 < SAS_MERGE_SYNC_WORDS) {
-        const int nblk = (L + s2b - 1) / s2b, bhi = p_hi < L ? j_end : nblk;
-        const int npc = split_arrive(a, slot0, slot, bhi - blo, bhi == nblk, nblk, &merge_word);
+      const bool cont = first_item && j_start > 0;
+      const int slot0 = cont ? slot - (cont_k < 0 ? -cont_k : cont_k) : slot;
+      if (split_slots_ok(a, slot0, slot)) {
+        const int npc = split_arrive(a, slot0, slot, cont && cont_k > 0, &merge_word);
         if (npc > 0) merge_item_here<DV, T, MB, NW>(a, tok, hb, slot0, npc);
       }
+      if (!cont) last_owed = false;
     }
     if (partial) ++slot;
-    if (is_end) break;
     first_item = false;
+    if (is_end) break;
     ++m;
   }
+  if (last_owed || (merge_here && first_item && j_start > 0))
+    split_settle(a, first_item && j_start > 0, cont_k, last_owed, slot);
   zero_unowned_rows<T>(a, tok_lo, tok_hi, fa_row, nfa, tid, NT);
 }
 

@@ -209,8 +209,18 @@ __global__ __launch_bounds__(512) void wide_kernel(const KernelArgs a) {
   const char* cmp_kv = (const char*)(a.cmp_kv ? a.cmp_kv : a.ori_kv);
   const float sc = a.softmax_scale * LOG2E;
   if (tid < 2) first_neg[tid] = INT32_MAX;
-  // piece index of the first item when it continues a split item
-  const int cont_k = (merge_here && j_start > 0) ? continued_piece_index(a, fa_row, b, m, cscan) : 0;
+  // piece index of the first item when it continues a split item, negative when the
+  // item goes on in the next row (by the schedule, whatever the lengths are by now);
+  // last_owed: the row's last piece, of an item that begins here, is not counted in
+  int cont_k = 0;
+  bool last_owed = merge_here && j_end > 0;
+  if (merge_here && j_start > 0) {
+    cont_k = continued_piece_index(a, fa_row, b, m, cscan);
+    if (j_end > 0 && b == b_end && m == s_end) {
+      cont_k = -cont_k;
+      last_owed = false;
+    }
+  }
   __syncthreads();
   // sink of this lane's head (an item holds every head: one head block)
   const float sink_h = hlocal < a.num_heads ? a.sinks[hlocal] : -INFINITY;
@@ -882,19 +892,22 @@ __global__ __launch_bounds__(512) void wide_kernel(const KernelArgs a) {
     if (partial && merge_here) {
       // the piece that completes the item merges it (bit-identical to merge_kernel)
       const KernelArgs a = fresh_args();
-      const int slot0 = (first_item && j_start > 0) ? slot - cont_k : slot;
-      if (slot0 >= 0 && slot < a.num_partial_slots && slot0 < SAS_MERGE_SYNC_WORDS) {
-        const int nblk = (L + s2b - 1) / s2b, bhi = p_hi < L ? j_end : nblk;
-        const int npc = split_arrive(a, slot0, slot, bhi - blo, bhi == nblk, nblk, &merge_word);
+      const bool cont = first_item && j_start > 0;
+      const int slot0 = cont ? slot - (cont_k < 0 ? -cont_k : cont_k) : slot;
+      if (split_slots_ok(a, slot0, slot)) {
+        const int npc = split_arrive(a, slot0, slot, cont && cont_k > 0, &merge_word);
         if (npc > 0) merge_item_here<DV, T, IMB, NW>(a, tok, hb, slot0, npc);
       }
+      if (!cont) last_owed = false;
     }
     if (partial) ++slot;
-    if (is_end) break;
     first_item = false;
+    if (is_end) break;
     if (pair) ++m;
     ++m;
   }
+  if (last_owed || (merge_here && first_item && j_start > 0))
+    split_settle(a, first_item && j_start > 0, cont_k, last_owed, slot);
   zero_unowned_rows<T>(a, tok_lo, tok_hi, fa_row, nfa, tid, NT);
 }
 
