@@ -280,18 +280,6 @@ __device__ __attribute__((aligned(256))) unsigned char g_zero_row[1152];
 
 // What the attention kernels are launched with: the call's arguments and the
 // divisors of the index arithmetic as multipliers.
-struct FastDiv {
-  uint32_t mul, shift;
-  // floor(n / d), 0 <= n < 2^31: with l = ceil(log2 d) and mul = ceil(2^(31 + l) / d),
-  // mul * d exceeds 2^(31 + l) by less than d <= 2^l, so n times the excess stays
-  // below 2^(31 + l) and the quotient exact
-  static FastDiv of(int d) {
-    uint32_t l = 0;
-    while (((int64_t)1 << l) < d) ++l;
-    return {(uint32_t)((((uint64_t)1 << (31 + l)) + (uint64_t)d - 1) / (uint64_t)d), l};
-  }
-  __device__ int div(int n) const { return (int)(__umulhi((uint32_t)n << 1, mul) >> shift); }
-};
 struct KernelArgs : SasAttnArgs {
   FastDiv ori_bs, cmp_bs, ratio;  // of the block sizes and cmp_ratio
 };
@@ -329,22 +317,8 @@ __device__ __forceinline__ KernelArgs fresh_args() {
   return a;
 }
 
-// item_geom (sas_items.h) of one item with the division by cmp_ratio as a product: an
-// item's last position + 1 never exceeds its length, so one at or below 0 is an item
-// that attends nothing.
 __device__ inline ItemGeom item_geom_at(const KernelArgs& a, int act_q, int act_kv, int s) {
-  const int64_t end64 = (int64_t)act_kv - act_q + s + 1;
-  const int end = end64 < 0 ? 0 : (end64 > INT32_MAX ? INT32_MAX : (int)end64);
-  ItemGeom g = {0, 0, 0, 0};
-  if (end > 0) {
-    g.win_lo = end - 1 >= a.ori_win_left ? end - 1 - a.ori_win_left : 0;
-    g.n_win = end - g.win_lo;
-  }
-  if (a.scenario >= 2) {
-    g.thr = a.ratio.div(end);
-    g.n_cmp = a.scenario == 3 && a.topk < g.thr ? a.topk : g.thr;
-  }
-  return g;
+  return item_geom_div(act_q, act_kv, s, a.ori_win_left, a.scenario, a.ratio, a.topk);
 }
 
 // Positions [c0, c0 + clen) of an item's list -> cache rows in LDS (rowid: row number,

@@ -53,4 +53,41 @@ __host__ __device__ inline ItemGeom item_geom(int32_t act_q, int32_t act_kv, int
   return g;
 }
 
+// Division by a number known at the launch, by multiplication.
+struct FastDiv {
+  uint32_t mul, shift;
+  // floor(n / d), 0 <= n < 2^31: with l = ceil(log2 d) and mul = ceil(2^(31 + l) / d),
+  // mul * d exceeds 2^(31 + l) by less than d <= 2^l, so n times the excess stays
+  // below 2^(31 + l) and the quotient exact
+  static FastDiv of(int d) {
+    uint32_t l = 0;
+    while (((int64_t)1 << l) < d) ++l;
+    return {(uint32_t)((((uint64_t)1 << (31 + l)) + (uint64_t)d - 1) / (uint64_t)d), l};
+  }
+  __host__ __device__ int div(int n) const {
+    return (int)((uint32_t)(((uint64_t)((uint32_t)n << 1) * mul) >> 32) >> shift);
+  }
+};
+
+// item_geom as the kernels form it for each item: in 32 bits, the division a product.
+// An item's last position + 1 never exceeds its length, so one at or below 0 is an item
+// that attends nothing, and every win_left below 0 is an empty window. The same as
+// item_geom for 0 <= s < act_q (win_lo only where there is a window).
+__host__ __device__ inline ItemGeom item_geom_div(int act_q, int act_kv, int s, int win_left,
+                                                  int scenario, FastDiv cmp_ratio, int topk) {
+  const int64_t end64 = (int64_t)act_kv - act_q + s + 1;
+  const int end = end64 < 0 ? 0 : (end64 > INT32_MAX ? INT32_MAX : (int)end64);
+  const int left = win_left < -1 ? -1 : win_left;
+  ItemGeom g = {0, 0, 0, 0};
+  if (end > 0) {
+    g.win_lo = end - 1 >= left ? end - 1 - left : 0;
+    g.n_win = end - g.win_lo;
+  }
+  if (scenario >= 2) {
+    g.thr = cmp_ratio.div(end);
+    g.n_cmp = scenario == 3 && topk < g.thr ? topk : g.thr;
+  }
+  return g;
+}
+
 }  // namespace sas
