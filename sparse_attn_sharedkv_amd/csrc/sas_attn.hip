@@ -211,20 +211,29 @@ struct QRows {
 };
 
 // Cumulative row counts: tokens outside [lo, hi) belong to no row of the schedule;
-// their output and lse rows are zeroed, spread over the workgroups in use (a fill of
-// every output row in front of the kernel took 12 us of a 128 x 128-head decode call).
+// their output and lse rows are zeroed, spread over the workgroups (a fill of every
+// output row in front of the kernel took 12 us of a 128 x 128-head decode call). A
+// launch may be for more FA rows than are in use: the shares of rows out of use go to
+// the row in use before them, those before any to the first.
 template <typename T>
 __device__ inline void zero_unowned_rows(const SasAttnArgs& a, int lo, int hi, int wg, int nwg,
                                          int tid, int nthreads) {
   lo = lo < 0 ? 0 : (lo < a.total_tokens ? lo : a.total_tokens);
   hi = hi < lo ? lo : (hi < a.total_tokens ? hi : a.total_tokens);
   const int n = lo + a.total_tokens - hi;
-  for (int r = wg; r < n; r += nwg) {
-    const size_t row = (size_t)(r < lo ? r : hi + r - lo) * a.num_heads;
-    i32x4* out = (i32x4*)((T*)a.out + row * a.head_dim_v);
-    for (int k = tid; k < a.num_heads * a.head_dim_v / 8; k += nthreads) out[k] = (i32x4){0, 0, 0, 0};
-    for (int k = tid; k < a.num_heads; k += nthreads) a.lse[row + k] = 0.0f;
-  }
+  if (n == 0) return;
+  auto out_of_use = [&](int row) { return a.metadata[row * SAS_FA_METADATA_SIZE] == 0; };
+  int first = wg, end = wg + 1;
+  while (end < nwg && out_of_use(end)) ++end;
+  while (first > 0 && out_of_use(first - 1)) --first;
+  if (first > 0) first = wg;
+  for (int share = first; share < end; ++share)
+    for (int r = share; r < n; r += nwg) {
+      const size_t row = (size_t)(r < lo ? r : hi + r - lo) * a.num_heads;
+      i32x4* out = (i32x4*)((T*)a.out + row * a.head_dim_v);
+      for (int k = tid; k < a.num_heads * a.head_dim_v / 8; k += nthreads) out[k] = (i32x4){0, 0, 0, 0};
+      for (int k = tid; k < a.num_heads; k += nthreads) a.lse[row + k] = 0.0f;
+    }
 }
 
 template <int N>
@@ -916,8 +925,7 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const KernelArgs a) {
   if (fa[0] == 0) return;
   // where the whole schedule ends (loaded beside this row's cursors)
   const int32_t* fa_last = a.metadata + (nfa - 1) * SAS_FA_METADATA_SIZE;
-  const int last_b = fa_last[4] < 0 ? 0 : (fa_last[4] < a.batch ? fa_last[4] : a.batch);
-  const int last_m = fa_last[4] < a.batch ? fa_last[5] : 0;
+  int last_on = fa_last[0], last_b = fa_last[4], last_m = fa_last[5];
   int b = fa[1], m = fa[2];
   const int j_start = fa[3];
   const int b_end = fa[4], s_end = fa[5], j_end = fa[6];
@@ -963,8 +971,14 @@ __global__ __launch_bounds__(128 * NHG) void attn2_kernel(const KernelArgs a) {
   // cumulative row counts: the tokens [tok_lo, tok_hi) of the schedule's rows
   int tok_lo = 0, tok_hi = a.total_tokens;
   if (qrows.cumulative) {
+    while (last_on == 0) {  // (a row out of use: the last one before it, at most this one)
+      fa_last -= SAS_FA_METADATA_SIZE;
+      last_on = fa_last[0], last_b = fa_last[4], last_m = fa_last[5];
+    }
     tok_lo = ld_uniform(qrows.first);
-    tok_hi = ld_uniform(qrows.first + last_b) + (last_m >> hshift);
+    const bool inside = last_b < a.batch;
+    tok_hi = ld_uniform(qrows.first + (last_b < 0 ? 0 : (inside ? last_b : a.batch))) +
+             (inside ? last_m >> hshift : 0);
   }
   int item_par = 0;  // which first_neg slot the next top-k scan uses
   bool first_item = true;
@@ -1684,8 +1698,7 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const KernelArgs a) {
   if (fa[0] == 0) return;
   // where the whole schedule ends (loaded beside this row's cursors)
   const int32_t* fa_last = a.metadata + (nfa - 1) * SAS_FA_METADATA_SIZE;
-  const int last_b = fa_last[4] < 0 ? 0 : (fa_last[4] < a.batch ? fa_last[4] : a.batch);
-  const int last_m = fa_last[4] < a.batch ? fa_last[5] : 0;
+  int last_on = fa_last[0], last_b = fa_last[4], last_m = fa_last[5];
   int b = fa[1], m = fa[2];
   const int j_start = fa[3];
   const int b_end = fa[4], s_end = fa[5], j_end = fa[6];
@@ -1704,8 +1717,14 @@ __global__ __launch_bounds__(256 * NHG) void attn3_kernel(const KernelArgs a) {
   // cumulative row counts: the tokens [tok_lo, tok_hi) of the schedule's rows
   int tok_lo = 0, tok_hi = a.total_tokens;
   if (qrows.cumulative) {
+    while (last_on == 0) {  // (a row out of use: the last one before it, at most this one)
+      fa_last -= SAS_FA_METADATA_SIZE;
+      last_on = fa_last[0], last_b = fa_last[4], last_m = fa_last[5];
+    }
     tok_lo = ld_uniform(qrows.first);
-    tok_hi = ld_uniform(qrows.first + last_b) + (last_m >> hshift);
+    const bool inside = last_b < a.batch;
+    tok_hi = ld_uniform(qrows.first + (last_b < 0 ? 0 : (inside ? last_b : a.batch))) +
+             (inside ? last_m >> hshift : 0);
   }
 
   // Sinks of this lane's softmax head in the (at most two) head blocks of an

@@ -192,8 +192,7 @@ __global__ __launch_bounds__(512) void wide_kernel(const KernelArgs a) {
   if (fa[0] == 0) return;
   // where the whole schedule ends (loaded beside this row's cursors)
   const int32_t* fa_last = a.metadata + (nfa - 1) * SAS_FA_METADATA_SIZE;
-  const int last_b = fa_last[4] < 0 ? 0 : (fa_last[4] < a.batch ? fa_last[4] : a.batch);
-  const int last_m = fa_last[4] < a.batch ? fa_last[5] : 0;
+  int last_on = fa_last[0], last_b = fa_last[4], last_m = fa_last[5];
   int b = fa[1], m = fa[2];
   const int j_start = fa[3];
   const int b_end = fa[4], s_end = fa[5], j_end = fa[6];
@@ -230,8 +229,14 @@ __global__ __launch_bounds__(512) void wide_kernel(const KernelArgs a) {
   // cumulative row counts: the tokens [tok_lo, tok_hi) of the schedule's rows
   int tok_lo = 0, tok_hi = a.total_tokens;
   if (qrows.cumulative) {
+    while (last_on == 0) {  // (a row out of use: the last one before it, at most this one)
+      fa_last -= SAS_FA_METADATA_SIZE;
+      last_on = fa_last[0], last_b = fa_last[4], last_m = fa_last[5];
+    }
     tok_lo = ld_uniform(qrows.first);
-    tok_hi = ld_uniform(qrows.first + last_b) + (last_m >> ((a.num_heads + IMB - 1) / IMB - 1));
+    const bool inside = last_b < a.batch;
+    tok_hi = ld_uniform(qrows.first + (last_b < 0 ? 0 : (inside ? last_b : a.batch))) +
+             (inside ? last_m >> ((a.num_heads + IMB - 1) / IMB - 1) : 0);
   }
   int item_par = 0;  // which first_neg slot the next top-k scan uses
   bool first_item = true;
