@@ -245,9 +245,10 @@ int sas_attention_launch(const SasAttnArgs* args, void* stream);
 int sas_attention_launch_lens(const SasAttnArgs* args, int q_lens, void* stream);
 
 /* Arrival counters (SasAttnArgs.merge_sync) for calls captured on `stream`, which must be
- * capturing: a zeroed array of the library's own, the same one for every call of one
- * capture on one stream. An array belongs to its capture's graph until the process ends;
- * NULL (see sas_last_error) once SAS_MERGE_SYNC_POOL arrays of the device are taken. */
+ * capturing: a zeroed array of the library's own, the same one as the call before got if
+ * that was for the same stream of the same capture, else the next. An array belongs to its
+ * capture's graph until the process ends; NULL (see sas_last_error) once
+ * SAS_MERGE_SYNC_POOL arrays of the device are taken. */
 #define SAS_MERGE_SYNC_POOL 1024
 uint64_t* sas_merge_sync_take(void* stream);
 

@@ -2844,7 +2844,8 @@ extern "C" uint64_t* sas_merge_sync_take(void* stream) {
     }
     p.base = (char*)at;
   }
-  // calls of one capture on one stream run one after another: they share an array
+  // calls of one capture on one stream run one after another, so they may share an
+  // array; those taken in turn with another stream's take more than one
   if (p.used == 0 || p.capture != capture || p.stream != (hipStream_t)stream) {
     if (p.used == SAS_MERGE_SYNC_POOL) {
       sas::set_error("sas_merge_sync_take: every array is taken");
