@@ -81,9 +81,13 @@ class Prepared:
 
 # Split items are merged inside the attention kernel (by the piece that finishes
 # last) when no item has more than this many pieces; with more, the merge kernel
-# spreads the merging over all compute units and is faster (measured on MI355X:
-# items of 2 pieces merge in ~2 us less inside the kernel; items of 8 pieces take
-# ~3 us longer there).
+# spreads the merging over all compute units and is faster, although it is a second
+# launch, or a second node of a graph. Measured on MI355X, us, merge kernel / inside,
+# replays of a graph of one call (calls in a row): MLA decode 64 x 128 heads, 2 pieces,
+# 69.2 / 66.6 (63.7 / 62.0); in 128-head items, 4 pieces, 70.2 / 70.9 (65.6 / 65.1);
+# window + top-k decode of 64 sequences, 3 pieces, 32.4 / 35.3 (28.0 / 30.5), of 32,
+# 5 pieces, 24.9 / 29.7 (20.6 / 25.0); MLA decode 32 x 128 heads, 8 pieces,
+# 50.8 / 55.5 (46.1 / 50.7).
 MERGE_IN_KERNEL_MAX_PIECES = 2
 
 
@@ -174,9 +178,9 @@ def _schedule_buffer(dev: torch.device) -> torch.Tensor:
 # Arrival counters of the split-KV merge done inside the attention kernel
 # (SasAttnArgs.merge_sync): zero at rest, one buffer per (device, stream) so that
 # calls on different streams never share one. Calls captured into a HIP graph take
-# one of the library's own zeroed arrays (sas_merge_sync_take: one per capture and
-# stream, taken for the life of the process); when those are all taken, a buffer
-# zeroed by a fill kernel recorded in the graph.
+# one of the library's own zeroed arrays (sas_merge_sync_take: calls that follow one
+# another on one stream of a capture share one, taken for the life of the process);
+# when those are all taken, a buffer zeroed by a fill kernel recorded in the graph.
 _MERGE_SYNC: dict = {}
 _CAPTURED_MERGE_SYNC: list = []
 

@@ -430,7 +430,9 @@ __global__ __launch_bounds__(NT) void sched_kernel(const Params p) {
     const Runs runs = {run_start, nblk, (int)num_runs};
     // (a budget never exceeds the total of all costs)
     const bool small = s_total < SMALL && p.min_split_blocks < SMALL;
-    // a walk has at most a step per run and per core: checkpoints cover all of it
+    // One lane's walk has at most a step per run and per core, and the stride spreads the
+    // checkpoints over as many; a wave walks each run until its slowest lane is through,
+    // so its walk may be longer, and what follows the last checkpoint is recorded from there
     const int steps = runs.num + p.num_cores + 1;
     const int stride = steps > 16 * NCK ? (steps + NCK - 1) / NCK : 16;
     auto clamp_ms = [&](int64_t ms) { return small && ms > SMALL ? SMALL : ms; };
